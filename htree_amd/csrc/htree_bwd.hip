@@ -35,6 +35,7 @@
 #include <mutex>
 
 #include "htree_common.h"
+#include "htree_tree_index.h"
 
 namespace htree {
 
@@ -414,8 +415,9 @@ __global__ __launch_bounds__(256) void pack_bwd_kernel(
   const int64_t tr = (bh * (Np / 16) + node / 16) * D * 16 + (dd >> 4) * 256 + (c >> 2) * 64 +
                      (dd & 15) * 4 + (c & 3);
   const int64_t vsrc = (bh * (Np / 16) + node / 16) * D * 16 + (c >> 2) * 4 * D + dd * 4 + (c & 3);
-  if (kt_h) kt_h[tr] = kh[idx];
-  if (kt_l) kt_l[tr] = kl[idx];
+  const int64_t ksrc = tree_kfrag(D, idx);
+  if (kt_h) kt_h[tr] = kh[ksrc];
+  if (kt_l) kt_l[tr] = kl[ksrc];
   if (vr_h) vr_h[idx] = vh[vsrc];
   if (vr_l) vr_l[idx] = vl[vsrc];
 }
@@ -448,7 +450,7 @@ __global__ __launch_bounds__(256) void pack_kt16_kernel(const uint16_t* __restri
     const int o = i * 64 + lane;
     const int d = (o >> 8) * 16 + ((o & 63) >> 2);
     const int c = ((o & 255) >> 6) * 4 + (o & 3);
-    const int64_t src = (row0 + c) * D + d;
+    const int64_t src = row0 * D + (d >> 3) * 128 + c * 8 + (d & 7);
     x[i] = bf_to_f(kh[src]) + bf_to_f(kl[src]);
     amax = fmaxf(amax, fabsf(x[i]));
   }
@@ -477,7 +479,7 @@ __global__ __launch_bounds__(256) void pack_vrot_kernel(
   const int64_t r = idx / half;  // bh * Np + node
   const int64_t node = r % Np;
   const int64_t a = ((node >> crlg) & vmask) << crlg;  // table row of the added angle
-  const int64_t e0 = r * D + i, e1 = e0 + half;
+  const int64_t e0 = tree_kfrag(D, r * D + i), e1 = tree_kfrag(D, r * D + i + half);
   const float x0 = bf_to_f(kh[e0]) + bf_to_f(kl[e0]);
   const float x1 = bf_to_f(kh[e1]) + bf_to_f(kl[e1]);
   const float c = cosb[a * half + i], sn = sinb[a * half + i];
@@ -764,7 +766,7 @@ __global__ __launch_bounds__(256) void record_wide_kernel(
 
 // ---------------------------------------------------------------- dkv
 struct DkvArgs {
-  const uint16_t *kh, *kl;      // K~ rows (hi/lo), [B][Hkv][Np][D]
+  const uint16_t *kh, *kl;      // K~ blocks (hi / lo) of the level (htree_common.h)
   const uint16_t *vt_h, *vt_l;  // the tree's V^T blocks (hi / lo) of the level
   const void* q;
   const void* dO;
@@ -1091,10 +1093,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // stationary K~ / V fragments of the tile's children (lane cand = u16)
   bf16x8 kh[KS], kl[KS], vh[KS], vl[KS];
   {
-    const int64_t r = (bh * a.Np + (live ? node0 : 0) + (u16 < CRU ? u16 : 0)) * D;
     if (!HAS_S) {  // K~ only rebuilds the scores
-      load_frag<D>(a.kh + r, kg, kh);
-      load_frag<D>(a.kl + r, kg, kl);
+      load_kfrag<D>(a.kh + bh * a.Np * D, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kh);
+      load_kfrag<D>(a.kl + bh * a.Np * D, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kl);
     }
     const int64_t vnode = (live ? node0 : 0) + (u16 < CRU ? u16 : 0);
     load_frag_vt<D>(a.vt_h, bh, a.Np, vnode, kg, vh);
@@ -1499,9 +1500,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   };
   bf16x8 kh[KS], kl[KS], vh[KS];
   {
-    const int64_t r = (bh * a.Np + (live ? node0 : 0) + (u16 < CRU ? u16 : 0)) * D;
-    load_frag<D>(a.kh + r, kg, kh);
-    load_frag<D>(a.kl + r, kg, kl);
+    load_kfrag<D>(a.kh + bh * a.Np * D, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kh);
+    load_kfrag<D>(a.kl + bh * a.Np * D, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kl);
     load_frag_vt<D>(a.vt_h, bh, a.Np, (live ? node0 : 0) + (u16 < CRU ? u16 : 0), kg, vh);
   }
   f32x4 dv[ND], dk[ND];
@@ -1932,9 +1932,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 32 ? 5
     auto kload = [&](int tau, bf16x8 (&kh)[KS], bf16x8 (&kl)[KS]) {
       const int posk = wide ? (tau << 4) + u16 : (tau << crlg) + u16;
       const bool cvk = u16 < CRU && posk < nc;
-      const int64_t krow = (hrow + node0_of(tau) + (cvk ? u16 : 0)) * D;
-      load_frag<D>(P.kh + krow, kg, kh);
-      load_frag<D>(P.kl + krow, kg, kl);
+      const int node0 = node0_of(tau), c = cvk ? u16 : 0;
+      load_kfrag<D>(P.kh + hrow * D, node0, c, kg, kh);
+      load_kfrag<D>(P.kl + hrow * D, node0, c, kg, kl);
     };
     // query frame of slot 0: angle apos
     float qr[KS][8];

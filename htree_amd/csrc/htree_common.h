@@ -41,7 +41,16 @@ constexpr int kSplitMaxTK = 2048;
 
 // ---------------------------------------------------------------- plan
 // Packed operand tree, per level l (all bf16, Np = N rounded up to 16):
-//   KH/KL [B][H_kv][Np][D]      hi / lo bf16 split of R(K_l[node], node mod CR)
+//   KH/KL [B][H_kv][Np/16][D/8][16][8]  hi / lo bf16 split of
+//                               R(K_l[node], node mod CR), in blocks of 16
+//                               nodes laid out as the MFMA operand reads them
+//                               (element (c, d) at (d/8)*128 + c*8 + d%8):
+//                               an operand load of a tile is 1 KB in a row.
+//                               With rows of 2 D bytes its lanes fell on 16
+//                               lines in 16-byte pieces, and the forwards were
+//                               bound by that L1 traffic: D 128, T 32768, 32/2
+//                               heads, 2.70 -> 1.94 ms; T 131072, 64/8 heads
+//                               (copies into LDS) 160 -> 143 ms.
 //   VH/VL [B][H_kv][Np/16][4][D][4]  V_l transposed in blocks of 16 nodes,
 //                               each block as four quads of 4 nodes
 //                               (element (d, c) at (c/4)*4D + d*4 + c%4)
@@ -536,12 +545,15 @@ struct LevelPtrs {
   int64_t N, Np, pw;
 };
 
-// The lane's K~ fragment of one candidate row (the lane group's d-slots).
+// The lane's K~ fragment of one candidate (the lane group's d-slots, chunk
+// 4 m + kg of the block layout above): node node0 + c of the (b, h_kv) at
+// base, in node0's block (a tile never crosses one).
 template <int D>
-__device__ __forceinline__ void load_kfrag(const uint16_t* __restrict__ row, int kg,
-                                           bf16x8 (&f)[D / 32]) {
+__device__ __forceinline__ void load_kfrag(const uint16_t* __restrict__ base, int node0, int c,
+                                           int kg, bf16x8 (&f)[D / 32]) {
+  const uint16_t* p = base + (int64_t)(node0 & ~15) * D + (((node0 & 15) + c) * 8 + kg * 128);
 #pragma unroll
-  for (int m = 0; m < D / 32; ++m) f[m] = *(const bf16x8*)(row + dslot<D>(kg, m));
+  for (int m = 0; m < D / 32; ++m) f[m] = *(const bf16x8*)(p + m * 512);
 }
 
 // exp(x) for x <= 0 (x = -inf gives 0) including subnormal results, which

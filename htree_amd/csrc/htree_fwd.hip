@@ -196,17 +196,15 @@ __device__ __forceinline__ float trace_merge(const FwdArgs& a, int64_t hq, bool 
   return gs;
 }
 
-// One tile's inputs staged in LDS: the K~ rows (hi, lo; each row padded by
-// 16 bytes, so that the 16 lanes reading one 16-byte column position of 16
-// rows hit distinct banks) and the tile's 16-node V^T block (hi, lo).
+// One tile's inputs staged in LDS: the 16-node K~ blocks (hi, lo) and the
+// V^T block (hi, lo) that hold the tile, as they lie in the packed tree (an
+// operand read's 64 lanes take 1 KB in a row: no bank conflicts).
 template <int D, bool PREC>
 struct FwdStage {
-  static constexpr int CPR = D * 2 / 16;          // 16-byte chunks of a K~ row
-  static constexpr int KRP = (CPR + 1) * 16;      // padded row pitch (bytes)
-  static constexpr int NCH = 16 * (CPR + 1);      // chunks of the 16 padded rows
-  static constexpr int OFF_KL = 16 * KRP;
+  static constexpr int KB = 16 * D * 2;           // K~ block of 16 nodes (bf16)
+  static constexpr int OFF_KL = KB;
   static constexpr int VB = 16 * D * 2;           // V^T block of 16 nodes (bf16)
-  static constexpr int OFF_V = 32 * KRP;
+  static constexpr int OFF_V = 2 * KB;
   static constexpr int OFF_VL = OFF_V + VB;
   static constexpr int BYTES = OFF_V + (PREC ? 2 : 1) * VB;
 };
@@ -225,17 +223,13 @@ struct TileStage {
   __device__ __forceinline__ void issue(int node0, bool with_v, int lane) const {
     int ln = lane;
     asm volatile("" : "+v"(ln));
+    const int koff = (node0 >> 4) * St::KB;
 #pragma unroll
-    for (int j = 0; j < (St::NCH + 63) / 64; ++j) {
-      const int pc = j * 64 + ln;
-      const int g = pc / (St::CPR + 1);
-      const int c = pc - g * (St::CPR + 1);
-      const int off = (node0 + g) * (D * 2) + (c < St::CPR ? c : 0) * 16;
-      if ((St::NCH % 64 == 0) || pc < St::NCH) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rkh, (lds_void*)(slot + j * 1024), 16, off, 0, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rkl, (lds_void*)(slot + St::OFF_KL + j * 1024), 16,
-                                                 off, 0, 0, 0);
-      }
+    for (int j = 0; j < St::KB / 1024; ++j) {
+      const int off = koff + (j * 64 + ln) * 16;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rkh, (lds_void*)(slot + j * 1024), 16, off, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rkl, (lds_void*)(slot + St::OFF_KL + j * 1024), 16,
+                                               off, 0, 0, 0);
     }
     if (with_v) {
       const int voff = (node0 >> 4) * St::VB;
@@ -257,15 +251,16 @@ struct TileStage {
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the slot's reads have completed
     __builtin_amdgcn_wave_barrier();
   }
-  // K~ fragments of row (candidate) u16, the lane group's d-slots
-  __device__ __forceinline__ void kread(bf16x8 (&kh)[D / 32], bf16x8 (&kl)[D / 32], int lane) const {
+  // K~ fragments of node c of the staged block, the lane group's d-slots
+  __device__ __forceinline__ void kread(bf16x8 (&kh)[D / 32], bf16x8 (&kl)[D / 32], int c,
+                                        int lane) const {
     int ln = lane;
     asm volatile("" : "+v"(ln));
-    const char* row = slot + (ln & 15) * St::KRP;
+    const char* row = slot + c * 16 + (ln >> 4) * 256;
 #pragma unroll
     for (int m = 0; m < D / 32; ++m) {
-      kh[m] = *(const bf16x8*)(row + dslot<D>(ln >> 4, m) * 2);
-      kl[m] = *(const bf16x8*)(row + St::OFF_KL + dslot<D>(ln >> 4, m) * 2);
+      kh[m] = *(const bf16x8*)(row + m * 1024);
+      kl[m] = *(const bf16x8*)(row + St::OFF_KL + m * 1024);
     }
   }
   // V^T fragments: nodes c0 .. c0+3 (one quad, c0 % 4 == 0) of the staged
@@ -400,7 +395,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     auto issue = [&](int tau, bool with_v) { stg.issue(node0_of(tau), with_v, lane); };
     auto wait_copies = [&]() { stg.wait_copies(); };
     auto reads_done = [&]() { stg.reads_done(); };
-    auto kread = [&](bf16x8 (&kh)[KS], bf16x8 (&kl)[KS]) { stg.kread(kh, kl, lane); };
+    // node of the staged block: the tile's candidate u16 (CR < 16: the
+    // tile starts inside the block)
+    auto kread = [&](int tau, bf16x8 (&kh)[KS], bf16x8 (&kl)[KS]) {
+      const int c = wide ? u16 : (node0_of(tau) & 15) + (u16 < CRU ? u16 : 0);
+      stg.kread(kh, kl, c, lane);
+    };
     // the query turned to a slot: R(q, apos) at slot 0, -CR per slot after
     float qr[KS][8];
     int cur_slot = 0;
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
         frame_to(slot_of(tau));
         wait_copies();
         bf16x8 kh[KS], kl[KS];
-        kread(kh, kl);
+        kread(tau, kh, kl);
         reads_done();
         if (tau + 1 < nt) issue(tau + 1, false);
         bf16x8 qh[KS], ql[KS];
@@ -559,7 +559,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       const unsigned long long smask = upper ? W.selmask[tau >> 2] : 0ull;
       wait_copies();
       bf16x8 kh[KS], kl[KS];
-      kread(kh, kl);
+      kread(tau, kh, kl);
       // V^T fragment: nodes node0 + 4kg + 0..3 of the staged block at d = 16n + u16
       const int c0 = (node0 & 15) + (4 * kg < CRU ? 4 * kg : 0);
       s16x4 vh[ND], vl[ND];
@@ -880,9 +880,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     auto kload = [&](int tau, bf16x8 (&kh)[KS], bf16x8 (&kl)[KS]) {
       const int posk = wide ? (tau << 4) + u16 : (tau << crlg) + u16;
       const bool cvk = u16 < CRU && posk < nc;
-      const int64_t krow = (int64_t)(node0_of(tau) + (cvk ? u16 : 0)) * D;
-      load_kfrag<D>(KH + krow, kg, kh);
-      load_kfrag<D>(KL + krow, kg, kl);
+      const int node0 = node0_of(tau), c = cvk ? u16 : 0;
+      load_kfrag<D>(KH, node0, c, kg, kh);
+      load_kfrag<D>(KL, node0, c, kg, kl);
     };
 
     // ---- scores of every tile (descending slot), S^T into LDS
@@ -1270,10 +1270,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 32 && 
         to_bf_split<D>(qr, qh, ql);
         const int pos = wide ? (tau << 4) + u16 : (tau << crlg) + u16;
         const bool cv = u16 < CRU && pos < nc;
-        const int64_t krow = (int64_t)(node0_of(tau) + (cv ? u16 : 0)) * D;
+        const int node0 = node0_of(tau), c = cv ? u16 : 0;
         bf16x8 kh[KS], kl[KS];
-        load_kfrag<D>(KH + krow, kg, kh);
-        load_kfrag<D>(KL + krow, kg, kl);
+        load_kfrag<D>(KH, node0, c, kg, kh);
+        load_kfrag<D>(KL, node0, c, kg, kl);
         f32x4 S = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int m = 0; m < KS; ++m) {
@@ -1363,10 +1363,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 32 && 
       to_bf_split<D>(qr, qh, ql);
       const int posk = wide ? (tau << 4) + u16 : (tau << crlg) + u16;
       const bool cvk = u16 < CRU && posk < nc;
-      const int64_t krow = (int64_t)(node0 + (cvk ? u16 : 0)) * D;
       bf16x8 kh[KS], kl[KS];
-      load_kfrag<D>(KH + krow, kg, kh);
-      load_kfrag<D>(KL + krow, kg, kl);
+      load_kfrag<D>(KH, node0, cvk ? u16 : 0, kg, kh);
+      load_kfrag<D>(KL, node0, cvk ? u16 : 0, kg, kl);
       f32x4 S = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int m = 0; m < KS; ++m) {

@@ -151,10 +151,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     const int pos = wide ? (tau << 4) + u16 : (tau << crlg) + u16;
     const bool cv = u16 < CRU && pos < nc;
     const int node0 = (pc[s] << crlg) + (wide ? ((tau << 4) & (CR - 1)) : 0);
-    const int64_t krow = (int64_t)(node0 + (cv ? u16 : 0)) * D;
     bf16x8 kh[KS], kl[KS];
-    load_kfrag<D>(KH + krow, kg, kh);
-    load_kfrag<D>(KL + krow, kg, kl);
+    load_kfrag<D>(KH, node0, cv ? u16 : 0, kg, kh);
+    load_kfrag<D>(KL, node0, cv ? u16 : 0, kg, kl);
     f32x4 S = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int m = 0; m < KS; ++m) {
@@ -364,10 +363,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       for (int m = 0; m < KS; ++m) split8(qr[m], qh[m], ql[m]);
       const int posk = wide ? (tau << 4) + u16 : (tau << crlg) + u16;
       const bool cvk = u16 < CRU && posk < nc;
-      const int64_t krow = (int64_t)(node0 + (cvk ? u16 : 0)) * D;
       bf16x8 kh[KS], kl[KS];
-      load_kfrag<D>(KH + krow, kg, kh);
-      load_kfrag<D>(KL + krow, kg, kl);
+      load_kfrag<D>(KH, node0, cvk ? u16 : 0, kg, kh);
+      load_kfrag<D>(KL, node0, cvk ? u16 : 0, kg, kl);
       f32x4 S = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int m = 0; m < KS; ++m) {

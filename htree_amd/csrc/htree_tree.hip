@@ -156,10 +156,11 @@ __device__ __forceinline__ void pack_k(const BuildArgs& a, int l, int64_t bh, in
                           r1[2 * q + 1] - __uint_as_float(h1[q] & 0xffff0000u));
     }
     const int64_t row = tree_krow(a.Np[l], D, bh, node);
-    *(uint2*)(kh + row + i0) = make_uint2(h0[0], h0[1]);
-    *(uint2*)(kh + row + HALF + i0) = make_uint2(h1[0], h1[1]);
-    *(uint2*)(kl + row + i0) = make_uint2(l0[0], l0[1]);
-    *(uint2*)(kl + row + HALF + i0) = make_uint2(l1[0], l1[1]);
+    const int64_t o0 = tree_kfrag(D, row + i0), o1 = tree_kfrag(D, row + HALF + i0);
+    *(uint2*)(kh + o0) = make_uint2(h0[0], h0[1]);
+    *(uint2*)(kh + o1) = make_uint2(h1[0], h1[1]);
+    *(uint2*)(kl + o0) = make_uint2(l0[0], l0[1]);
+    *(uint2*)(kl + o1) = make_uint2(l1[0], l1[1]);
   }
 }
 
@@ -216,9 +217,9 @@ __device__ __forceinline__ void zero_padding(const BuildArgs& a, int64_t bh) {
     for (int it = threadIdx.x; it < np * D; it += blockDim.x) {
       const int j = it / D, d = it - j * D;
       const int64_t node = a.N[l] + j;
-      const int64_t row = tree_krow(a.Np[l], D, bh, node);
-      a.kh[l][row + d] = 0;
-      a.kl[l][row + d] = 0;
+      const int64_t ko = tree_kfrag(D, tree_krow(a.Np[l], D, bh, node) + d);
+      a.kh[l][ko] = 0;
+      a.kl[l][ko] = 0;
       const int64_t o = vt_index(a, l, bh, node, d);
       a.vh[l][o] = 0;
       if (a.vl[l]) a.vl[l][o] = 0;

@@ -47,6 +47,17 @@ __host__ __device__ inline int64_t tree_krow(int64_t Np, int D, int64_t bh, int6
   return (bh * Np + node) * D;
 }
 
+// Where element r of that row-major numbering (r = krow + d) lies in the K~
+// arrays: 16-node blocks in MFMA operand order, 8-element chunks of the 16
+// nodes one after the other, element (c, d) of a block at
+// (d / 8) * 128 + c * 8 + d % 8, so that the 64 lanes of an operand load
+// (16 nodes x 4 chunks) read 1 KB in a row.
+__host__ __device__ inline int64_t tree_kfrag(int D, int64_t r) {
+  const int64_t n = r / D;
+  const int d = (int)(r - n * D), c = (int)(n & 15);
+  return (n - c) * D + (d >> 3) * 128 + c * 8 + (d & 7);
+}
+
 // Element (d, node) of a level's V^T blocks: 16-node blocks of four 4-node
 // quads, (d, c) at (c / 4) * 4D + d * 4 + c % 4.
 __host__ __device__ inline int64_t tree_vt_index(int64_t Np, int D, int64_t bh, int64_t node,

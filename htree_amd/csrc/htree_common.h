@@ -158,6 +158,10 @@ template <>
 struct Io<float> {
   static __device__ __forceinline__ float ld(const float* p) { return *p; }
   static __device__ __forceinline__ void st(float* p, float v) { *p = v; }
+  static __device__ __forceinline__ void st8(float* p, const float* v) {
+    *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
+    *(float4*)(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+  }
   static __device__ __forceinline__ void ld8(const float* p, float* o) {
     float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
     o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w;
@@ -168,6 +172,11 @@ template <>
 struct Io<__bf16> {
   static __device__ __forceinline__ float ld(const __bf16* p) { return (float)*p; }
   static __device__ __forceinline__ void st(__bf16* p, float v) { *p = (__bf16)v; }
+  static __device__ __forceinline__ void st8(__bf16* p, const float* v) {
+    typedef __attribute__((ext_vector_type(8))) float f8;
+    const f8 x = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+    *(bf16x8*)p = __builtin_convertvector(x, bf16x8);
+  }
   static __device__ __forceinline__ void ld8(const __bf16* p, float* o) {
     uint4 r = *(const uint4*)p;
     uint32_t w[4] = {r.x, r.y, r.z, r.w};
@@ -182,6 +191,12 @@ template <>
 struct Io<_Float16> {
   static __device__ __forceinline__ float ld(const _Float16* p) { return (float)*p; }
   static __device__ __forceinline__ void st(_Float16* p, float v) { *p = (_Float16)v; }
+  static __device__ __forceinline__ void st8(_Float16* p, const float* v) {
+    typedef __attribute__((ext_vector_type(8))) float f8;
+    typedef __attribute__((ext_vector_type(8))) _Float16 h8;
+    const f8 x = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+    *(h8*)p = __builtin_convertvector(x, h8);
+  }
   static __device__ __forceinline__ void ld8(const _Float16* p, float* o) {
     typedef __attribute__((ext_vector_type(8))) _Float16 h8;
     h8 r = *(const h8*)p;

@@ -450,7 +450,7 @@ __global__ __launch_bounds__(256) void pack_kt16_kernel(const uint16_t* __restri
     const int o = i * 64 + lane;
     const int d = (o >> 8) * 16 + ((o & 63) >> 2);
     const int c = ((o & 255) >> 6) * 4 + (o & 3);
-    const int64_t src = row0 * D + (d >> 3) * 128 + c * 8 + (d & 7);
+    const int64_t src = tree_kfrag(D, (row0 + c) * D + d);
     x[i] = bf_to_f(kh[src]) + bf_to_f(kl[src]);
     amax = fmaxf(amax, fabsf(x[i]));
   }
@@ -985,9 +985,15 @@ __device__ __forceinline__ void ld_chunk<float>(const float* p, float* o) {
   o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w;
 }
 
-// Row fragment (head u16, the lane group's d-slots) of the staged rows
-template <int D, typename TIn>
+// Row fragment (head u16) of the staged rows: the lane group's d-slots, or
+// with PAIRS K~'s operand order (query rows)
+template <int D, typename TIn, bool PAIRS = false>
 __device__ __forceinline__ void row_frag(const char* rows, int u16, int kg, float (&x)[D / 32][8]) {
+  if constexpr (PAIRS && D == 32) {
+    Io<TIn>::ld4((const TIn*)(rows + row_off<D, TIn>(u16, 4 * kg)), x[0]);
+    Io<TIn>::ld4((const TIn*)(rows + row_off<D, TIn>(u16, 16 + 4 * kg)), x[0] + 4);
+    return;
+  }
   constexpr int PER = 16 / (int)sizeof(TIn);  // elements per chunk
 #pragma unroll
   for (int m = 0; m < D / 32; ++m) {
@@ -1217,7 +1223,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       // rotated query fragment (lane g = u16); the score scale is applied to S
       // (heads past the group hold finite filler: their P and dS are zeroed below)
       float qr[KS][8];
-      row_frag<D, TIn>(S0, u16, kg, qr);
+      row_frag<D, TIn, true>(S0, u16, kg, qr);
       rot_by_fr<D>(qr, tab, tab + HALF, kg);
       bf16x8 qh[KS], ql[KS];
       split_frag<D>(qr, qh, ql);
@@ -1572,7 +1578,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     f32x4 S = {0.f, 0.f, 0.f, 0.f};
     {
       float qr[KS][8];
-      row_frag<D, __bf16>(S0, u16, kg, qr);
+      row_frag<D, __bf16, true>(S0, u16, kg, qr);
       const float* tq = u16 < 8 ? tab0 : tab1;
       rot_by_fr<D>(qr, tq, tq + HALF, kg);
       bf16x8 qh[KS], ql[KS];
@@ -1950,8 +1956,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 32 ? 5
       // that tile's MFMAs)
 #pragma unroll
       for (int m = 0; m < KS; ++m) {
-        *(bf16x8*)(KTh + u16 * KRP + dslot<D>(kg, m) * 2) = kh[m];
-        *(bf16x8*)(KTl + u16 * KRP + dslot<D>(kg, m) * 2) = kl[m];
+        if constexpr (D == 32) {  // (pairs 4 kg .. 4 kg + 3: two pieces)
+          const uint4 wh = __builtin_bit_cast(uint4, kh[m]), wl = __builtin_bit_cast(uint4, kl[m]);
+          *(uint2*)(KTh + u16 * KRP + 8 * kg) = make_uint2(wh.x, wh.y);
+          *(uint2*)(KTh + u16 * KRP + 32 + 8 * kg) = make_uint2(wh.z, wh.w);
+          *(uint2*)(KTl + u16 * KRP + 8 * kg) = make_uint2(wl.x, wl.y);
+          *(uint2*)(KTl + u16 * KRP + 32 + 8 * kg) = make_uint2(wl.z, wl.w);
+        } else {
+          *(bf16x8*)(KTh + u16 * KRP + dslot<D>(kg, m) * 2) = kh[m];
+          *(bf16x8*)(KTl + u16 * KRP + dslot<D>(kg, m) * 2) = kl[m];
+        }
       }
       const int s = wide ? (tau << 4) >> crlg : tau;
       if (s != cur_slot) {  // ascending slots, one step apart

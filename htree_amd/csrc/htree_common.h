@@ -44,7 +44,8 @@ constexpr int kSplitMaxTK = 2048;
 //   KH/KL [B][H_kv][Np/16][D/8][16][8]  hi / lo bf16 split of
 //                               R(K_l[node], node mod CR), in blocks of 16
 //                               nodes laid out as the MFMA operand reads them
-//                               (element (c, d) at (d/8)*128 + c*8 + d%8):
+//                               (element (c, d) at (d/8)*128 + c*8 + d%8;
+//                               D = 32: d in pair order, tree_kfrag):
 //                               an operand load of a tile is 1 KB in a row.
 //                               With rows of 2 D bytes its lanes fell on 16
 //                               lines in 16-byte pieces, and the forwards were
@@ -57,6 +58,13 @@ constexpr int kSplitMaxTK = 2048;
 // Scores always use the split product (plain bf16 scores err by ~2e-2 when
 // |q||k| is large, e.g. clustered keys); VL exists for fp32/fp16 inputs only
 // (bf16 V is exact in VH).
+//   SH/SL                     D = 32: the same K~ with d in dslot's order, which
+//                               the scores that select are summed in (every
+//                               level; levels >= 1 for the wide forward).
+//                               D >= 64: KH/KL, where the two orders agree.
+//   AH/AL (wide forward)        the top level's R(K, node): its candidates are
+//                               nodes 0 .. t's, so the accumulation there meets
+//                               them with one turn of the query for the level.
 // Rows >= N of the padding are zero.
 struct Plan {
   int L;
@@ -66,6 +74,8 @@ struct Plan {
   int64_t pw[HTREE_MAX_LEVELS];  // CR^l
   int64_t off_kh[HTREE_MAX_LEVELS], off_kl[HTREE_MAX_LEVELS];
   int64_t off_vh[HTREE_MAX_LEVELS], off_vl[HTREE_MAX_LEVELS];
+  int64_t off_sh[HTREE_MAX_LEVELS], off_sl[HTREE_MAX_LEVELS];  // -1: none
+  int64_t off_ah, off_al;                                      // -1: none
   int64_t bytes;
   int max_tiles;  // candidate tiles of 16 per level: TK * max(CR,16) / 16
   int cr_log2;
@@ -162,6 +172,10 @@ struct Io<float> {
     *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
     *(float4*)(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
   }
+  static __device__ __forceinline__ void ld4(const float* p, float* o) {
+    const float4 a = *(const float4*)p;
+    o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w;
+  }
   static __device__ __forceinline__ void ld8(const float* p, float* o) {
     float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
     o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w;
@@ -176,6 +190,13 @@ struct Io<__bf16> {
     typedef __attribute__((ext_vector_type(8))) float f8;
     const f8 x = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
     *(bf16x8*)p = __builtin_convertvector(x, bf16x8);
+  }
+  static __device__ __forceinline__ void ld4(const __bf16* p, float* o) {
+    const uint2 r = *(const uint2*)p;
+    o[0] = __uint_as_float(r.x << 16);
+    o[1] = __uint_as_float(r.x & 0xffff0000u);
+    o[2] = __uint_as_float(r.y << 16);
+    o[3] = __uint_as_float(r.y & 0xffff0000u);
   }
   static __device__ __forceinline__ void ld8(const __bf16* p, float* o) {
     uint4 r = *(const uint4*)p;
@@ -196,6 +217,12 @@ struct Io<_Float16> {
     typedef __attribute__((ext_vector_type(8))) _Float16 h8;
     const f8 x = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
     *(h8*)p = __builtin_convertvector(x, h8);
+  }
+  static __device__ __forceinline__ void ld4(const _Float16* p, float* o) {
+    typedef __attribute__((ext_vector_type(4))) _Float16 h4;
+    const h4 r = *(const h4*)p;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = (float)r[i];
   }
   static __device__ __forceinline__ void ld8(const _Float16* p, float* o) {
     typedef __attribute__((ext_vector_type(8))) _Float16 h8;
@@ -318,6 +345,7 @@ __device__ __forceinline__ int add_xor32i(int x) {
   const auto r = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
   return (int)r[0] + (int)r[1];
 }
+
 // x of lane ^ 32
 __device__ __forceinline__ float xor32(float x) {
   float a, b;
@@ -357,39 +385,47 @@ __device__ __forceinline__ int mbcnt64(unsigned long long m) {
 }
 
 // d-slot of k-step m for lane group kg: the four lane groups cover 8
-// consecutive elements each; steps m and m + D/64 hold the RoPE pair
-// (d, d + D/2) so both halves of a pair live in the same lane.  D = 32 has
-// one k-step: lane groups 0, 1 hold the low half, 2, 3 the high half, and a
-// pair's halves sit in lanes 32 apart.
+// consecutive elements each.  The operand order of V and dO.
 template <int D>
 __device__ __forceinline__ int dslot(int kg, int m) {
+  return 8 * kg + 32 * m;
+}
+
+// The pair order of K~ (KH / KL) and of the queries it meets holds both
+// halves (d, d + D/2) of a RoPE pair in one lane: D >= 64 in k-steps m and
+// m + D/64 of dslot's order; D = 32, which has one k-step, the pairs
+// 4 kg .. 4 kg + 3 in elements e (d = 4 kg + e) and e + 4 (d = 16 + 4 kg + e).
+// In dslot's order at D = 32 a pair's halves sit 32 lanes apart and every turn
+// of a query pays 8 lane swaps: the backward's dkv at top_k 512, T 12000,
+// 64/4 heads, fp32 takes 11.1 ms with them and 10.2 without, its dq 7.3 and
+// 6.1.
+template <int D, typename TIn>
+__device__ __forceinline__ void ld_pairs(const TIn* p, int kg, int m, float* o) {
   if constexpr (D == 32) {
-    return 8 * kg;
+    Io<TIn>::ld4(p + 4 * kg, o);
+    Io<TIn>::ld4(p + 16 + 4 * kg, o + 4);
   } else {
-    constexpr int SPH = D / 64;
-    return 8 * kg + 32 * (m % SPH) + (D / 2) * (m / SPH);
+    Io<TIn>::ld8(p + dslot<D>(kg, m), o);
   }
 }
 
-// y = R(x, p) on an operand fragment laid out by dslot (R of
-// src/naive.py:22-28: lo' = lo cos - hi sin, hi' = lo sin + hi cos), with
-// cosr / sinr the table row of angle p.  x and y may alias.
+// y = R(x, p) on a fragment in pair order (R of src/naive.py:22-28:
+// lo' = lo cos - hi sin, hi' = lo sin + hi cos), with cosr / sinr the table
+// row of angle p.  x and y may alias.
 template <int D>
 __device__ __forceinline__ void rope_frag(const float (&x)[D / 32][8], const float* __restrict__ cosr,
                                           const float* __restrict__ sinr, int kg,
                                           float (&y)[D / 32][8]) {
   if constexpr (D == 32) {
-    float c[8], s[8], t[8];
-    Io<float>::ld8(cosr + 8 * (kg & 1), c);
-    Io<float>::ld8(sinr + 8 * (kg & 1), s);
-    const float sg = kg < 2 ? -1.f : 1.f;  // lo lanes subtract hi sin, hi lanes add lo sin
+    float c[4], s[4];
+    Io<float>::ld4(cosr + 4 * kg, c);
+    Io<float>::ld4(sinr + 4 * kg, s);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float other = xor32(x[0][e]);
-      t[e] = x[0][e] * c[e] + sg * other * s[e];
+    for (int e = 0; e < 4; ++e) {
+      const float lo = x[0][e], hi = x[0][e + 4];
+      y[0][e] = lo * c[e] - hi * s[e];
+      y[0][e + 4] = lo * s[e] + hi * c[e];
     }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) y[0][e] = t[e];
   } else {
     constexpr int SPH = D / 64;
 #pragma unroll
@@ -428,7 +464,8 @@ __device__ __forceinline__ int row_sum16i(int x) {
 // Block-wide Top-K of a block of kWideWaves waves: thread i holds the keys of
 // positions C*i .. C*i+C-1 in registers (key 0 = no candidate; a larger key
 // is a larger value).  select() finds the `take` largest keys with a bitwise
-// radix select from bit `top_bit` down (per step: a per-lane count, a DPP row
+// radix select from bit `top_bit` down, ending at the first bit that leaves
+// exactly `take` keys (per step: a per-lane count, a DPP row
 // sum and one block barrier; the reduction slots alternate, so a slot is
 // rewritten only after every wave has passed the barrier that follows its
 // last read), gives the ties at the threshold to the lowest positions (the
@@ -448,17 +485,20 @@ struct BlockSelect {
   }
   int32_t* red;
   int lane, wv;
+  bool has = true;  // the wave holds any key (wave-uniform)
   int rc = 0, rs = 0;
 
   __device__ __forceinline__ int count(const uint32_t (&key)[C], uint32_t thr, bool strict) {
     int c = 0;
+    if (has) {
 #pragma unroll
-    for (int i = 0; i < C; ++i) {
-      c += strict ? key[i] > thr : key[i] >= thr;
-      if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // keep the compare masks short-lived
+      for (int i = 0; i < C; ++i) {
+        c += strict ? key[i] > thr : key[i] >= thr;
+        if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // keep the compare masks short-lived
+      }
+      c = row_sum16i(c);
+      c = add_xor32i(add_xor16i(c));
     }
-    c = row_sum16i(c);
-    c = add_xor32i(add_xor16i(c));
     int32_t* r = red + S * rc;
     rc ^= 1;
     if (lane == 0) r[wv] = c;
@@ -490,7 +530,9 @@ struct BlockSelect {
 #pragma unroll 1
     for (int bit = top_bit; bit >= 0; --bit) {
       const uint32_t c = thr | (1u << bit);
-      if (count(key, c, false) >= take) thr = c;
+      const int n = count(key, c, false);
+      if (n >= take) thr = c;
+      if (n == take) break;  // exactly the keys >= c: no tie to settle
     }
     const int need = take - count(key, thr, true);
     Mask gtb = 0, eqb = 0;  // this thread's positions above / at the threshold
@@ -508,15 +550,49 @@ struct BlockSelect {
   }
 };
 
-// Query fragment of a lane (head u16, the lane group's d-slots) kept in its
+// y = R(x, p) on a D = 32 fragment in dslot's order: a pair's halves sit in
+// lanes 32 apart.
+__device__ __forceinline__ void rope_frag32_lanes(const float (&x)[1][8],
+                                                  const float* __restrict__ cosr,
+                                                  const float* __restrict__ sinr, int kg,
+                                                  float (&y)[1][8]) {
+  float c[8], s[8], t[8];
+  Io<float>::ld8(cosr + 8 * (kg & 1), c);
+  Io<float>::ld8(sinr + 8 * (kg & 1), s);
+  const float sg = kg < 2 ? -1.f : 1.f;  // lo lanes subtract hi sin, hi lanes add lo sin
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float other = xor32(x[0][e]);
+    t[e] = x[0][e] * c[e] + sg * other * s[e];
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[0][e] = t[e];
+}
+
+// The turn in the order of the scores that select (dslot's).
+template <int D>
+__device__ __forceinline__ void rope_frag_s(const float (&x)[D / 32][8],
+                                            const float* __restrict__ cosr,
+                                            const float* __restrict__ sinr, int kg,
+                                            float (&y)[D / 32][8]) {
+  if constexpr (D == 32)
+    rope_frag32_lanes(x, cosr, sinr, kg, y);
+  else
+    rope_frag<D>(x, cosr, sinr, kg, y);
+}
+
+// Query fragment of a lane (head u16, pair order or with PAIRS = false dslot's) kept in its
 // input type; get() returns it in fp32 times `scale`.
-template <int D, typename TIn>
+template <int D, typename TIn, bool PAIRS = true>
 struct QFrag {
   float f[D / 32][8];
   __device__ __forceinline__ void load(const TIn* p, int kg, bool gv) {
 #pragma unroll
     for (int m = 0; m < D / 32; ++m) {
-      Io<TIn>::ld8(p + dslot<D>(kg, m), f[m]);
+      if constexpr (PAIRS)
+        ld_pairs<D, TIn>(p, kg, m, f[m]);
+      else
+        Io<TIn>::ld8(p + dslot<D>(kg, m), f[m]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) f[m][e] = gv ? f[m][e] : 0.f;
     }
@@ -528,13 +604,19 @@ struct QFrag {
       for (int e = 0; e < 8; ++e) x[m][e] = f[m][e] * scale;
   }
 };
-template <int D>
-struct QFrag<D, __bf16> {
+template <int D, bool PAIRS>
+struct QFrag<D, __bf16, PAIRS> {
   uint4 w[D / 32];  // 8 bf16 per k-step, exact
   __device__ __forceinline__ void load(const __bf16* p, int kg, bool gv) {
 #pragma unroll
     for (int m = 0; m < D / 32; ++m) {
-      const uint4 r = *(const uint4*)(p + dslot<D>(kg, m));
+      uint4 r;
+      if constexpr (PAIRS && D == 32) {
+        const uint2 lo = *(const uint2*)(p + 4 * kg), hi = *(const uint2*)(p + 16 + 4 * kg);
+        r = make_uint4(lo.x, lo.y, hi.x, hi.y);
+      } else {
+        r = *(const uint4*)(p + dslot<D>(kg, m));
+      }
       w[m] = gv ? r : make_uint4(0u, 0u, 0u, 0u);
     }
   }
@@ -557,6 +639,8 @@ struct LevelPtrs {
   const uint16_t* kl;
   const uint16_t* vh;
   const uint16_t* vl;
+  const uint16_t* sh;  // wide forward: K~ of the scores that select
+  const uint16_t* sl;
   int64_t N, Np, pw;
 };
 

@@ -1,0 +1,6 @@
+// Wide forward, head dim 32.
+#include "htree_fwd_wide.h"
+
+namespace htree {
+template void launch_fwd_wide_d<32>(int dtype, const FwdArgs& a, dim3 grid, hipStream_t st, bool sel);
+}  // namespace htree

@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     const int s = wide ? (tau << 4) >> crlg : tau;
     const int prow = apos - (s << crlg);
     float qr[KS][8];
-    rope_frag<D>(qf, a.cosb + (int64_t)prow * HALF, a.sinb + (int64_t)prow * HALF, kg, qr);
+    rope_frag_s<D>(qf, a.cosb + (int64_t)prow * HALF, a.sinb + (int64_t)prow * HALF, kg, qr);
     bf16x8 qh[KS], ql[KS];
 #pragma unroll
     for (int m = 0; m < KS; ++m) split8(qr[m], qh[m], ql[m]);
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       }
       if (!any) continue;  // every candidate of the tile passed down
       float qr[KS][8];
-      rope_frag<D>(qf, a.cosb + (int64_t)prow * HALF, a.sinb + (int64_t)prow * HALF, kg, qr);
+      rope_frag_s<D>(qf, a.cosb + (int64_t)prow * HALF, a.sinb + (int64_t)prow * HALF, kg, qr);
       bf16x8 qh[KS], ql[KS];
 #pragma unroll
       for (int m = 0; m < KS; ++m) split8(qr[m], qh[m], ql[m]);
@@ -568,8 +568,8 @@ int split_forward(const htree_dims* d, const Plan& P, float scale, const void* q
   memset(&a, 0, sizeof(a));
   const char* base = (const char*)tree_ws;
   for (int l = 0; l < P.L; ++l) {
-    a.lv[l].kh = (const uint16_t*)(base + P.off_kh[l]);
-    a.lv[l].kl = P.off_kl[l] >= 0 ? (const uint16_t*)(base + P.off_kl[l]) : nullptr;
+    a.lv[l].kh = (const uint16_t*)(base + P.off_sh[l]);
+    a.lv[l].kl = (const uint16_t*)(base + P.off_sl[l]);
     a.lv[l].vh = (const uint16_t*)(base + P.off_vh[l]);
     a.lv[l].vl = P.off_vl[l] >= 0 ? (const uint16_t*)(base + P.off_vl[l]) : nullptr;
     a.lv[l].N = P.N[l];

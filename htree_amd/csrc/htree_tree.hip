@@ -72,6 +72,7 @@ int make_plan(const htree_dims* d, Plan* p) {
   if (!tree_level_sizes(d->T, CR, d->max_top_nodes, HTREE_MAX_LEVELS, p->N, &L))
     return HTREE_EUNSUPPORTED;
   p->L = L;
+  const bool wide_fwd = (wide || d->kv_share == 4) && !split;
   int64_t off = 0, pw = 1;
   const int64_t BH = (int64_t)d->B * d->H_kv;
   auto take = [&](int64_t elems) {
@@ -88,7 +89,16 @@ int make_plan(const htree_dims* d, Plan* p) {
     p->off_kl[l] = take(elems);
     p->off_vh[l] = take(elems);
     p->off_vl[l] = p->precise ? take(elems) : -1;
+    p->off_sh[l] = p->off_kh[l];
+    p->off_sl[l] = p->off_kl[l];
+    if (d->D == 32) {
+      const bool selects = l > 0 || !wide_fwd;  // (the register forward scores every level once)
+      p->off_sh[l] = selects ? take(elems) : -1;
+      p->off_sl[l] = selects ? take(elems) : -1;
+    }
   }
+  p->off_ah = wide_fwd ? take(BH * p->Np[L - 1] * d->D) : -1;
+  p->off_al = wide_fwd ? take(BH * p->Np[L - 1] * d->D) : -1;
   p->bytes = off;
   // one (b, h_kv) block of a level's operand arrays is addressed through a
   // buffer resource of 32-bit range
@@ -115,6 +125,9 @@ struct BuildArgs {
   uint16_t* kl[HTREE_MAX_LEVELS];
   uint16_t* vh[HTREE_MAX_LEVELS];
   uint16_t* vl[HTREE_MAX_LEVELS];       // nullptr for bf16 inputs
+  uint16_t* sh[HTREE_MAX_LEVELS];       // D = 32: K~ in dslot's order (or nullptr)
+  uint16_t* sl[HTREE_MAX_LEVELS];
+  uint16_t *ah, *al;                    // top level's K at the angle of its node (or nullptr)
   int64_t N[HTREE_MAX_LEVELS], Np[HTREE_MAX_LEVELS], pw[HTREE_MAX_LEVELS];
   const float *cosb, *sinb;
   int64_t chunks;                       // spans per (b, h_kv)
@@ -124,19 +137,22 @@ struct BuildArgs {
 // K~ of nodes nf .. nf+cnt-1 of level l: R(K, node mod CR) split into bf16
 // hi / lo; val(j, e) is element e of node nf + j.  A thread takes 4
 // consecutive RoPE pairs (i, i + D/2) of one node (8-byte stores).
+// `abs`: R(K, node) into the top level's own arrays.
 template <typename F>
-__device__ __forceinline__ void pack_k(const BuildArgs& a, int l, int64_t bh, int64_t nf, int cnt,
-                                       F val) {
+__device__ __forceinline__ void pack_k_at(const BuildArgs& a, int l, int64_t bh, int64_t nf, int cnt,
+                                          bool abs, F val) {
   const int D = a.D, HALF = D / 2, Q = D / 8;
-  uint16_t* kh = a.kh[l];
-  uint16_t* kl = a.kl[l];
+  uint16_t* kh = abs ? a.ah : a.kh[l];
+  uint16_t* kl = abs ? a.al : a.kl[l];
+  uint16_t* sh = abs ? nullptr : a.sh[l];
+  uint16_t* sl = a.sl[l];
   for (int it = threadIdx.x; it < cnt * Q; it += blockDim.x) {
     int j, i0;
     pack_k_item(it, D, &j, &i0);
     const int64_t node = nf + j;
-    const int c = (int)(node & (a.CR - 1));
-    const float* cr = a.cosb + (int64_t)c * HALF + i0;
-    const float* sr = a.sinb + (int64_t)c * HALF + i0;
+    const int64_t c = abs ? node : node & (a.CR - 1);
+    const float* cr = a.cosb + c * HALF + i0;
+    const float* sr = a.sinb + c * HALF + i0;
     float r0[4], r1[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -161,7 +177,20 @@ __device__ __forceinline__ void pack_k(const BuildArgs& a, int l, int64_t bh, in
     *(uint2*)(kh + o1) = make_uint2(h1[0], h1[1]);
     *(uint2*)(kl + o0) = make_uint2(l0[0], l0[1]);
     *(uint2*)(kl + o1) = make_uint2(l1[0], l1[1]);
+    if (sh) {
+      const int64_t s0 = tree_kchunk(D, row + i0), s1 = tree_kchunk(D, row + HALF + i0);
+      *(uint2*)(sh + s0) = make_uint2(h0[0], h0[1]);
+      *(uint2*)(sh + s1) = make_uint2(h1[0], h1[1]);
+      *(uint2*)(sl + s0) = make_uint2(l0[0], l0[1]);
+      *(uint2*)(sl + s1) = make_uint2(l1[0], l1[1]);
+    }
   }
+}
+template <typename F>
+__device__ __forceinline__ void pack_k(const BuildArgs& a, int l, int64_t bh, int64_t nf, int cnt,
+                                       F val) {
+  pack_k_at(a, l, bh, nf, cnt, false, val);
+  if (a.ah && l == a.L - 1) pack_k_at(a, l, bh, nf, cnt, true, val);
 }
 
 // element (d, node) of the level's V^T blocks
@@ -220,6 +249,15 @@ __device__ __forceinline__ void zero_padding(const BuildArgs& a, int64_t bh) {
       const int64_t ko = tree_kfrag(D, tree_krow(a.Np[l], D, bh, node) + d);
       a.kh[l][ko] = 0;
       a.kl[l][ko] = 0;
+      if (a.sh[l]) {
+        const int64_t so = tree_kchunk(D, tree_krow(a.Np[l], D, bh, node) + d);
+        a.sh[l][so] = 0;
+        a.sl[l][so] = 0;
+      }
+      if (a.ah && l == a.L - 1) {
+        a.ah[ko] = 0;
+        a.al[ko] = 0;
+      }
       const int64_t o = vt_index(a, l, bh, node, d);
       a.vh[l][o] = 0;
       if (a.vl[l]) a.vl[l][o] = 0;
@@ -377,9 +415,17 @@ static int tree_build_t(const htree_dims* d, const Plan& P, const void* k, const
     a.kl[l] = (uint16_t*)(base + P.off_kl[l]);
     a.vh[l] = (uint16_t*)(base + P.off_vh[l]);
     a.vl[l] = P.off_vl[l] >= 0 ? (uint16_t*)(base + P.off_vl[l]) : nullptr;
+    if (d->D == 32 && P.off_sh[l] >= 0) {
+      a.sh[l] = (uint16_t*)(base + P.off_sh[l]);
+      a.sl[l] = (uint16_t*)(base + P.off_sl[l]);
+    }
     a.N[l] = P.N[l];
     a.Np[l] = P.Np[l];
     a.pw[l] = P.pw[l];
+  }
+  if (P.off_ah >= 0) {
+    a.ah = (uint16_t*)(base + P.off_ah);
+    a.al = (uint16_t*)(base + P.off_al);
   }
   a.cosb = cosb;
   a.sinb = sinb;

@@ -52,10 +52,21 @@ __host__ __device__ inline int64_t tree_krow(int64_t Np, int D, int64_t bh, int6
 // nodes one after the other, element (c, d) of a block at
 // (d / 8) * 128 + c * 8 + d % 8, so that the 64 lanes of an operand load
 // (16 nodes x 4 chunks) read 1 KB in a row.
-__host__ __device__ inline int64_t tree_kfrag(int D, int64_t r) {
+__host__ __device__ inline int64_t tree_kchunk(int D, int64_t r) {
   const int64_t n = r / D;
   const int d = (int)(r - n * D), c = (int)(n & 15);
   return (n - c) * D + (d >> 3) * 128 + c * 8 + (d & 7);
+}
+// The same with both halves of a RoPE pair in one lane's chunks: D >= 64 the
+// order above; D = 32, whose one k-step would hold them 32 lanes apart, takes
+// d in the order of pair_slot32 (chunk kg: pairs 4 kg .. 4 kg + 3).
+__host__ __device__ inline int pair_slot32(int d) {
+  return ((d & 15) >> 2) * 8 + (d >> 4) * 4 + (d & 3);
+}
+__host__ __device__ inline int64_t tree_kfrag(int D, int64_t r) {
+  if (D != 32) return tree_kchunk(D, r);
+  const int64_t n = r / D;
+  return tree_kchunk(D, n * D + pair_slot32((int)(r - n * D)));
 }
 
 // Element (d, node) of a level's V^T blocks: 16-node blocks of four 4-node

@@ -1,5 +1,5 @@
-"""The packed K~ layout (tree_kfrag of htree_tree_index.h, which the build's
-stores and the operand reads share) on the CPU: within each block of 16 nodes
+"""The packed K~ layouts (tree_kfrag and tree_kchunk of htree_tree_index.h, which
+the build's stores and the operand reads share) on the CPU: within each block of 16 nodes
 a permutation of the row-major elements, 4 consecutive d stay together (the
 build's 8-byte stores), and lane (u16, kg) of operand load m reads 16 bytes at
 1 KB * m + 16 * lane (load_kfrag)."""
@@ -14,15 +14,18 @@ SRC = r'''
 using namespace htree;
 int main() {
   int bad = 0;
-  for (int D : {32, 64, 128, 256}) {
+  for (int D : {32, 64, 128, 256}) for (int pairs : {0, 1}) {
+    auto kfrag = [&](int64_t r) { return pairs ? tree_kfrag(D, r) : tree_kchunk(D, r); };
     std::vector<int> seen(48 * D, 0);
     for (int64_t n = 0; n < 48; ++n)
       for (int d = 0; d < D; ++d) {
-        const int64_t o = tree_kfrag(D, tree_krow(48, D, 0, n) + d);
+        const int64_t o = kfrag(tree_krow(48, D, 0, n) + d);
         if (o < n / 16 * 16 * D || o >= (n / 16 + 1) * 16 * D) ++bad; else ++seen[o];
-        const int m = d / 32, kg = d % 32 / 8, lane = kg * 16 + (int)(n % 16);
-        if (o != n / 16 * 16 * D + m * 512 + lane * 8 + d % 8) ++bad;
-        if (d % 4 && o != tree_kfrag(D, tree_krow(48, D, 0, n) + d - 1) + 1) ++bad;
+        // D = 32 in pair order: a lane holds both halves of RoPE pairs 4 kg .. 4 kg + 3
+        const int m = d / 32, kg = pairs && D == 32 ? d % 16 / 4 : d % 32 / 8, lane = kg * 16 + (int)(n % 16);
+        const int e = pairs && D == 32 ? d / 16 * 4 + d % 4 : d % 8;
+        if (o != n / 16 * 16 * D + m * 512 + lane * 8 + e) ++bad;
+        if (d % 4 && o != kfrag(tree_krow(48, D, 0, n) + d - 1) + 1) ++bad;
       }
     for (int s : seen) bad += s != 1;
   }

@@ -1,5 +1,5 @@
 // Arguments and device helpers shared by the fused forward kernels
-// (htree_fwd.hip, htree_fwd_stream.hip, htree_fwd_wide.hip).
+// (htree_fwd.hip, htree_fwd_stream.hip, htree_fwd_wide.h).
 #pragma once
 
 #include "htree_common.h"
@@ -8,6 +8,7 @@ namespace htree {
 
 // max of a level that accumulated nothing (src/naive.py:9, src/parallel.py:75)
 constexpr float kNegInfSentinel = -1.0e10f;
+constexpr float kLn2 = 0.69314718055994531f;
 
 struct FwdArgs {
   LevelPtrs lv[HTREE_MAX_LEVELS];

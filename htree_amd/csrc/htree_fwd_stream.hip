@@ -111,6 +111,12 @@ struct TileStage {
 // tau is computed.  Tiles run in ascending parent slot and the query turns
 // by R(., -CR) per slot (a table row in LDS), so a tile reads no global
 // memory besides its copies.
+// Bound by its vector ALU work per tile (T 131072, 64/8 heads, D 128, CR 32):
+// the turned query is split once per slot instead of once per tile, the
+// subnormal test is one per tile, a tile's masks are formed only at a level's
+// last tile, the passed-down candidates start their scores at -inf, and the
+// rescale runs only where a head's max rises: 132.1 -> 124.4 ms (same start,
+// 150.3 and 152.1 ms).
 template <int D, bool PREC, typename TIn, int MAXSLOT, bool TRACE, bool SEL = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void fwd_kernel(const FwdArgs a) {
   static_assert(!(SEL && TRACE), "selection only: no trace");
@@ -168,9 +174,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // query fragment (lane: head u16, the lane group's d-slots), kept in its
   // input type (16-bit types packed)
   QFrag<D, TIn, false> qin;
+  // Rows past the group repeat its heads: their scores stay in the range of
+  // the others, and they are left out of the sums and not stored.  (A padded
+  // group's are zero and masked, as its padding heads.)
   {
     const bool gv = u16 < G;
-    qin.load((const TIn*)a.q + (((int64_t)b * a.T + t) * a.H + h * G + (gv ? u16 : 0)) * D, kg, gv);
+    qin.load((const TIn*)a.q +
+                 (((int64_t)b * a.T + t) * a.H + h * G + (gv ? u16 : a.gpad > 0 ? 0 : u16 % G)) * D,
+             kg, gv || a.gpad == 0);
   }
 
   float m_run = -INFINITY, l_part = 0.f;
@@ -218,25 +229,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       const int c = wide ? u16 : (node0_of(tau) & 15) + (u16 < CRU ? u16 : 0);
       stg.kread(kh, kl, c, lane);
     };
-    // the query turned to a slot: R(q, apos) at slot 0, -CR per slot after
+    // the query turned to a slot, R(q, apos) at slot 0, -CR per slot after,
+    // and split once per slot (a slot has CR / 16 tiles; at D >= 128 with fp32
+    // or fp16 inputs once per tile, as the registers do not hold both)
+    constexpr bool ONCE = D <= 64 || !PREC;
     float qr[KS][8];
+    bf16x8 qh[KS], ql[KS];
     int cur_slot = 0;
-    auto frame_start = [&]() {
-      qin.get(qr, a.scale);
+    auto frame_start = [&](float scale) {
+      qin.get(qr, scale);
       rot_by<D>(qr, a.cosb + (int64_t)apos * HALF, a.sinb + (int64_t)apos * HALF, kg);
+      if (ONCE) to_bf_split<D>(qr, qh, ql);
       cur_slot = 0;
     };
     auto frame_to = [&](int s) {
-      while (cur_slot < s) {
+      if (cur_slot < s) {  // (tiles are taken in order: one slot on)
         rot_by<D>(qr, rot_m[0], rot_m[1], kg);
-        ++cur_slot;
+        if (ONCE) to_bf_split<D>(qr, qh, ql);
+        cur_slot = s;
       }
+      if (!ONCE) to_bf_split<D>(qr, qh, ql);
     };
 
     // ------------------------------------------------ selection (upper levels)
     if (upper) {
       float Mrun = -INFINITY;
-      frame_start();
+      float hm[4];  // 1 for heads 4kg + r of the selection (formed per level)
+      f32x4 hinit;
+      {
+        int kq = kg;
+        asm volatile("" : "+v"(kq));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          hm[r] = 4 * kq + r < Gs ? 1.f : 0.f;
+          hinit[r] = 4 * kq + r < Gs || a.gpad == 0 ? 0.f : -INFINITY;
+        }
+      }
+      frame_start(a.scale);
       issue(0, false);
       for (int tau = 0; tau < nt; ++tau) {
         frame_to(slot_of(tau));
@@ -245,11 +274,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
         kread(tau, kh, kl);
         reads_done();
         if (tau + 1 < nt) issue(tau + 1, false);
-        bf16x8 qh[KS], ql[KS];
-        to_bf_split<D>(qr, qh, ql);
-        const int pos = wide ? (tau << 4) + u16 : (tau << crlg) + u16;
-        const bool cv = u16 < CRU && pos < nc;
-        f32x4 S = {0.f, 0.f, 0.f, 0.f};
+        f32x4 S = hinit;
 #pragma unroll
         for (int m = 0; m < KS; ++m) {
           S = mma32(qh[m], kh[m], S);
@@ -257,16 +282,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
           S = mma32(ql[m], kh[m], S);
         }
         // S[r] = score[g = 4kg + r][candidate u16]
-        float tm = -INFINITY;
+        if (!wide || tau == nt - 1) {
+          const int pos = wide ? (tau << 4) + u16 : (tau << crlg) + u16;
+          const bool cv = u16 < CRU && pos < nc;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (cv && 4 * kg + r < Gs) tm = fmaxf(tm, S[r]);
-        tm = wave_max(tm);
-        Mrun = fmaxf(Mrun, tm);
+          for (int r = 0; r < 4; ++r) S[r] = cv ? S[r] : -INFINITY;
+        }
+        Mrun = fmaxf(Mrun, wave_max(fmaxf(fmaxf(S[0], S[1]), fmaxf(S[2], S[3]))));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[r] = (S[r] - Mrun) * kLog2e;
+        // subnormal results (exp_sel), one wave test for the tile
+        if (__builtin_expect(__any(fminf(fminf(S[0], S[1]), fminf(S[2], S[3])) < -126.f), 0)) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const bool sb = S[r] < -126.f;
+            const float p = __builtin_amdgcn_exp2f(sb ? S[r] + 64.f : S[r]);
+            S[r] = sb ? p * 5.42101086242752217e-20f : p;
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[r] = __builtin_amdgcn_exp2f(S[r]);
+        }
         float e = 0.f;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (cv && 4 * kg + r < Gs) e += exp_sel(S[r] - Mrun);
+        for (int r = 0; r < 4; ++r) e = fmaf(S[r], hm[r], e);
         e = add_xor32(add_xor16(e));
         if (kg == 0) W.imp[(tau << 4) + u16] = e;
         if (lane == 0) W.mt[tau] = Mrun;
@@ -368,12 +407,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
 #pragma unroll
       for (int n = 0; n < ND; ++n) O[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    frame_start();
+    // scores in log2 units (the query carries log2 e)
+    frame_start(a.scale * kLog2e);
     issue(0, true);
     for (int tau = 0; tau < nt; ++tau) {
       frame_to(slot_of(tau));
       const int node0 = node0_of(tau);
-      const unsigned long long smask = upper ? W.selmask[tau >> 2] : 0ull;
+      // -inf where the candidate is passed down
+      f32x4 S = {0.f, 0.f, 0.f, 0.f};
+      if (upper) {
+        const int w = uniform((int)(W.selmask[tau >> 2] >> (16 * (tau & 3))));
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          S[r] = __int_as_float(__builtin_amdgcn_sbfe(w, 4 * kg + r, 1) & 0xff800000);
+      }
       wait_copies();
       bf16x8 kh[KS], kl[KS];
       kread(tau, kh, kl);
@@ -383,37 +430,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       stg.vread(vh, vl, c0, u16);
       reads_done();
       if (tau + 1 < nt) issue(tau + 1, true);
-      bf16x8 qh[KS], ql[KS];
-      to_bf_split<D>(qr, qh, ql);
-      f32x4 S = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int m = 0; m < KS; ++m) {
         S = mma32(kh[m], qh[m], S);
         S = mma32(kl[m], qh[m], S);
         S = mma32(kh[m], ql[m], S);
       }
-      // S[r] = score[candidate 4kg + r][g = u16]
-      float sv[4];
+      // S[r] = log2 e score[candidate 4kg + r][g = u16]
+      if (!wide || tau == nt - 1) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int cu = 4 * kg + r;
-        const int pos = wide ? (tau << 4) + cu : (tau << crlg) + cu;
-        const bool ok = cu < CRU && pos < nc && !((smask >> ((16 * (tau & 3) + cu) & 63)) & 1ull);
-        sv[r] = ok ? S[r] : -INFINITY;
+        for (int r = 0; r < 4; ++r) {
+          const int cu = 4 * kg + r;
+          const int pos = wide ? (tau << 4) + cu : (tau << crlg) + cu;
+          S[r] = cu < CRU && pos < nc ? S[r] : -INFINITY;
+        }
       }
-      float tm = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
+      float tm = fmaxf(fmaxf(S[0], S[1]), fmaxf(S[2], S[3]));
       tm = max_xor32(max_xor16(tm));
       if (!__any(tm > -INFINITY)) continue;  // every candidate of the tile passed down
-      const float mnew = fmaxf(m_run, tm);
-      const float mref = mnew == -INFINITY ? 0.f : mnew;
-      const float alpha = __builtin_amdgcn_exp2f((m_run - mref) * kLog2e);
-      m_run = mnew;
+      if (__any(tm > m_run)) {  // some head's max rises: rescale
+        const float mnew = fmaxf(m_run, tm);
+        const float alpha = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - mnew);
+        m_run = mnew;
+        l_part *= alpha;
+#pragma unroll
+        for (int n = 0; n < ND; ++n) O[n] *= alpha;
+      }
+      const float mref = m_run == -INFINITY ? 0.f : m_run;
       float p[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f((sv[r] - mref) * kLog2e);
-      l_part = l_part * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
-#pragma unroll
-      for (int n = 0; n < ND; ++n) O[n] *= alpha;
+      for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(S[r] - mref);
+      l_part += (p[0] + p[1]) + (p[2] + p[3]);
       s16x4 ph, pl;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -432,14 +479,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     }
     wait_copies();  // no copy into the slot is left in flight past the level
     if (TRACE)
-      trace_store<D, true>(a, l, ((int64_t)b * a.T + t) * a.H + h * G + u16, u16 < G, kg, m_run,
-                           l_part, O);
+      trace_store<D, true>(a, l, ((int64_t)b * a.T + t) * a.H + h * G + u16, u16 < G, kg,
+                           m_run * kLn2, l_part, O);
     cur ^= 1;
   }
 
   if constexpr (SEL) return;
   // final normalisation (src/parallel.py:321-363): out = o / s
   float lt;
+  if (!TRACE) m_run *= kLn2;  // (natural units; the trace's states are)
   if (TRACE) {
     lt = trace_merge<D, true>(a, ((int64_t)b * a.T + t) * a.H + h * G + u16, u16 < G, kg, m_run, O);
   } else {

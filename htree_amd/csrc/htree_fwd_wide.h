@@ -46,8 +46,6 @@ namespace htree {
 // sum_i imp_i e^{m_i - M} (the group-shared sum over all of the group's
 // heads), and every part takes its result.
 
-constexpr float kLn2 = 0.69314718055994531f;
-
 // Reduces four values per lane (tile j in x_j) over the four lane groups:
 // lane group j ends with op over the groups of x_j, (g0 op g1) op (g2 op g3).
 template <typename Op>

@@ -220,7 +220,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
 
   // the query stays in its input type (16-bit types packed: 16 registers)
   QFrag<D, TIn, false> qin;
-  qin.load((const TIn*)a.q + (((int64_t)b * a.T + t) * a.H + h * G + (gv ? u16 : 0)) * D, kg, gv);
+  // rows past the group repeat its heads: their scores stay in the range of
+  // the others, and they are left out of the sums (hv) and not stored
+  qin.load((const TIn*)a.q + (((int64_t)b * a.T + t) * a.H + h * G + (gv ? u16 : u16 % G)) * D, kg, true);
+  const float hv = gv ? 1.f : 0.f;
 
   float m_run = -INFINITY, l_part = 0.f;
   f32x4 O[ND];
@@ -292,14 +295,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
         S = mma32(kl[m], qh[m], S);
         S = mma32(kh[m], ql[m], S);
       }
+      if (!wide || tau == nt - 1) {  // the other tiles hold 16 candidates
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int cu = 4 * kg + r;
-        const int pos = wide ? (tau << 4) + cu : (tau << crlg) + cu;
-        const bool ok = gv && cu < CRU && pos < nc;
-        S[r] = ok ? S[r] : -INFINITY;
-        lmax = fmaxf(lmax, S[r]);
+        for (int r = 0; r < 4; ++r) {
+          const int cu = 4 * kg + r;
+          const int pos = wide ? (tau << 4) + cu : (tau << crlg) + cu;
+          S[r] = cu < CRU && pos < nc ? S[r] : -INFINITY;
+        }
       }
+      lmax = fmaxf(lmax, fmaxf(fmaxf(S[0], S[1]), fmaxf(S[2], S[3])));
       W.st[tau][lane] = S;
     };
     for (int tau = nt - 1; tau >= 0; --tau) {
@@ -325,6 +329,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
           for (int r = 0; r < 4; ++r)
             if (x[r] < -126.f) e[r] = __builtin_amdgcn_exp2f(x[r] + 64.f) * 5.42101086242752217e-20f;
         }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) e[r] *= hv;
         // sum over the row's 16 lanes (heads) of each candidate r, by
         // recursive halving: lane bit 0 keeps r in {0,1} or {2,3}, bit 1 one
         // of those, then the four quads add up; lane u16 ends with candidate
@@ -366,10 +372,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     auto masked = [&](int tau) {
       f32x4 S = W.st[tau][lane];
       if (upper) {
-        const unsigned long long sm = W.selmask[tau >> 2];
+        const int w = uniform((int)(W.selmask[tau >> 2] >> (16 * (tau & 3))));
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if ((sm >> ((16 * (tau & 3) + 4 * kg + r) & 63)) & 1ull) S[r] = -INFINITY;
+        for (int r = 0; r < 4; ++r) {  // -inf where the candidate is passed down
+          const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe(w, 4 * kg + r, 1);
+          S[r] = __uint_as_float((m & 0xff800000u) | (~m & __float_as_uint(S[r])));
+        }
       }
       return S;
     };

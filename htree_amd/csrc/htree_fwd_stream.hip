@@ -171,18 +171,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   const int CRU = CR < 16 ? CR : 16;
   const bool wide = CR >= 16;
 
-  // query fragment (lane: head u16, the lane group's d-slots), kept in its
-  // input type (16-bit types packed)
-  QFrag<D, TIn, false> qin;
-  // Rows past the group repeat its heads: their scores stay in the range of
-  // the others, and they are left out of the sums and not stored.  (A padded
-  // group's are zero and masked, as its padding heads.)
-  {
-    const bool gv = u16 < G;
-    qin.load((const TIn*)a.q +
-                 (((int64_t)b * a.T + t) * a.H + h * G + (gv ? u16 : a.gpad > 0 ? 0 : u16 % G)) * D,
-             kg, gv || a.gpad == 0);
-  }
+  // Query rows past the group repeat its heads: their scores stay in the
+  // range of the others, and they are left out of the sums and not stored.  (A
+  // padded group's are zero and masked, as its padding heads.)
+  const bool gv = u16 < G;
+  const TIn* qp = (const TIn*)a.q +
+                  (((int64_t)b * a.T + t) * a.H + h * G + (gv ? u16 : a.gpad > 0 ? 0 : u16 % G)) * D;
 
   float m_run = -INFINITY, l_part = 0.f;
   f32x4 O[ND];
@@ -230,13 +224,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       stg.kread(kh, kl, c, lane);
     };
     // the query turned to a slot, R(q, apos) at slot 0, -CR per slot after,
-    // and split once per slot (a slot has CR / 16 tiles; at D >= 128 with fp32
-    // or fp16 inputs once per tile, as the registers do not hold both)
-    constexpr bool ONCE = D <= 64 || !PREC;
+    // and split once per slot (a slot has CR / 16 tiles; at D = 256 once per
+    // tile, as the registers do not hold both)
+    constexpr bool ONCE = D <= 128;
     float qr[KS][8];
     bf16x8 qh[KS], ql[KS];
     int cur_slot = 0;
     auto frame_start = [&](float scale) {
+      // (read again at each pass: held, its registers spill at D = 128)
+      QFrag<D, TIn, false> qin;
+      qin.load(qp, kg, gv || a.gpad == 0);
       qin.get(qr, scale);
       rot_by<D>(qr, a.cosb + (int64_t)apos * HALF, a.sinb + (int64_t)apos * HALF, kg);
       if (ONCE) to_bf_split<D>(qr, qh, ql);

@@ -230,11 +230,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     float qr[KS][8];
     bf16x8 qh[KS], ql[KS];
     int cur_slot = 0;
-    auto frame_start = [&](float scale) {
+    auto frame_start = [&]() {
       // (read again at each pass: held, its registers spill at D = 128)
       QFrag<D, TIn, false> qin;
       qin.load(qp, kg, gv || a.gpad == 0);
-      qin.get(qr, scale);
+      qin.get(qr, a.scale);
       rot_by<D>(qr, a.cosb + (int64_t)apos * HALF, a.sinb + (int64_t)apos * HALF, kg);
       if (ONCE) to_bf_split<D>(qr, qh, ql);
       cur_slot = 0;
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
           hinit[r] = 4 * kq + r < Gs || a.gpad == 0 ? 0.f : -INFINITY;
         }
       }
-      frame_start(a.scale);
+      frame_start();
       issue(0, false);
       for (int tau = 0; tau < nt; ++tau) {
         frame_to(slot_of(tau));
@@ -404,8 +404,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
 #pragma unroll
       for (int n = 0; n < ND; ++n) O[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    // scores in log2 units (the query carries log2 e)
-    frame_start(a.scale * kLog2e);
+    frame_start();
     issue(0, true);
     for (int tau = 0; tau < nt; ++tau) {
       frame_to(slot_of(tau));
@@ -433,7 +432,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
         S = mma32(kl[m], qh[m], S);
         S = mma32(kh[m], ql[m], S);
       }
-      // S[r] = log2 e score[candidate 4kg + r][g = u16]
+      // S[r] = score[candidate 4kg + r][g = u16]
       if (!wide || tau == nt - 1) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -445,19 +444,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       float tm = fmaxf(fmaxf(S[0], S[1]), fmaxf(S[2], S[3]));
       tm = max_xor32(max_xor16(tm));
       if (!__any(tm > -INFINITY)) continue;  // every candidate of the tile passed down
+      float alpha = 1.f;
       if (__any(tm > m_run)) {  // some head's max rises: rescale
         const float mnew = fmaxf(m_run, tm);
-        const float alpha = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - mnew);
+        alpha = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((m_run - mnew) * kLog2e);
         m_run = mnew;
-        l_part *= alpha;
 #pragma unroll
         for (int n = 0; n < ND; ++n) O[n] *= alpha;
       }
       const float mref = m_run == -INFINITY ? 0.f : m_run;
       float p[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(S[r] - mref);
-      l_part += (p[0] + p[1]) + (p[2] + p[3]);
+      for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f((S[r] - mref) * kLog2e);
+      l_part = l_part * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
       s16x4 ph, pl;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -477,14 +476,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     wait_copies();  // no copy into the slot is left in flight past the level
     if (TRACE)
       trace_store<D, true>(a, l, ((int64_t)b * a.T + t) * a.H + h * G + u16, u16 < G, kg,
-                           m_run * kLn2, l_part, O);
+                           m_run, l_part, O);
     cur ^= 1;
   }
 
   if constexpr (SEL) return;
   // final normalisation (src/parallel.py:321-363): out = o / s
   float lt;
-  if (!TRACE) m_run *= kLn2;  // (natural units; the trace's states are)
   if (TRACE) {
     lt = trace_merge<D, true>(a, ((int64_t)b * a.T + t) * a.H + h * G + u16, u16 < G, kg, m_run, O);
   } else {

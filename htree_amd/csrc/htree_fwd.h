@@ -8,7 +8,6 @@ namespace htree {
 
 // max of a level that accumulated nothing (src/naive.py:9, src/parallel.py:75)
 constexpr float kNegInfSentinel = -1.0e10f;
-constexpr float kLn2 = 0.69314718055994531f;
 
 struct FwdArgs {
   LevelPtrs lv[HTREE_MAX_LEVELS];

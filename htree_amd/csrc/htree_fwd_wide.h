@@ -29,8 +29,7 @@ namespace htree {
 //     (a skipped rescale where no head's max rises).  The top level's
 //     candidates are nodes 0 .. t's, met at R(K, node) with one turn of the
 //     query; below, the query takes a batch's last slot from the table and
-//     turns by CR per slot.  Scores are in log2 units (the query carries
-//     log2 e).
+//     turns by CR per slot.
 // Each wave keeps its own softmax state; they are merged at the end.
 // D = 32 is bound by the vector data path (72% busy: 2.0 TB of operands a
 // launch at T 120000, 64/4 heads, top_k 512) beside 59% of the vector ALU:
@@ -174,7 +173,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
         for (int w = 0; w < NW; ++w) {
           const float mw_ = mw[w * 16 + u16];
           if (mw_ == -INFINITY) continue;
-          const float sc = exp2f(mw_ - M);
+          const float sc = expf(mw_ - M);
           L += lw[w * 16 + u16] * sc;
 #pragma unroll
           for (int n = 0; n < ND; ++n)
@@ -182,7 +181,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
             for (int r = 0; r < 4; ++r) Om[n][r] += ow[(w * 16 + u16) * DP + 16 * n + 4 * kg + r] * sc;
         }
       }
-      Mo = M * kLn2;  // (natural units; -inf stays)
+      Mo = M;
       Lo = L;
     }
   };
@@ -452,7 +451,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
     for (int m = 0; m < KS; ++m) {
       ld_pairs<D, TIn>(qp, kg, m, qf[m]);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) qf[m][e] = zero_row ? 0.f : qf[m][e] * (a.scale * kLog2e);
+      for (int e = 0; e < 8; ++e) qf[m][e] = zero_row ? 0.f : qf[m][e] * a.scale;
     }
     bf16x8 qh[KS], ql[KS];
     if (top) {
@@ -568,7 +567,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
         int nn[UA];
         nodes(last || bi + NW >= nb ? bi : bi + NW, nn);
         if (PIPE) keys(nn);
-        // S[j][r] = log2 e score[candidate 4kg + r of tile tau0 + j][g = u16]
+        // S[j][r] = score[candidate 4kg + r of tile tau0 + j][g = u16]
         if ((FORM != 0 && !wide) || last) {
 #pragma unroll
           for (int j = 0; j < UA; ++j)
@@ -587,7 +586,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
         tm = max_xor32(max_xor16(tm));
         if (__any(tm > m_run)) {
           const float mnew = fmaxf(m_run, tm);
-          const float alpha = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - mnew);
+          const float alpha = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((m_run - mnew) * kLog2e);
           m_run = mnew;
           l_part *= alpha;
 #pragma unroll
@@ -602,7 +601,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
           }
           float p[4];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(S[j][r] - mref);
+          for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f((S[j][r] - mref) * kLog2e);
           l_part += (p[0] + p[1]) + (p[2] + p[3]);
           const uint32_t h01 = cvt_pk_bf16(p[0], p[1]), h23 = cvt_pk_bf16(p[2], p[3]);
           const s16x4 ph = __builtin_bit_cast(s16x4, make_uint2(h01, h23));

@@ -78,7 +78,8 @@ struct BwdPlan {
   int64_t off_vlist;                   // the merged level's lists [B,T,H_kv,TK]
   // the merged level's K~ rows (hi, lo) turned from the angle of the node's
   // child index (node mod CR) to that of its index in the 64-child parent
-  // (node mod 64), for a backward that rebuilds the scores (or -1)
+  // (node mod 64), for a backward that rebuilds the scores (or -1; none
+  // where the level's K~ is at the angle of the node)
   int64_t off_vk[2];
   // stored-dS path: each level's piece offsets / table / count of its own,
   // so that every level's index can be built ahead of the dK / dV passes
@@ -218,7 +219,7 @@ static int make_bwd_plan(const htree_dims* d, BwdPlan* b, bool allow_ds = true, 
   b->off_npieces = take(4);
   b->off_ptab = take(b->max_pieces * 3 * 4);
   b->off_vlist = b->vlevel >= 0 ? take(b->max_entries * 4) : -1;
-  if (b->vlevel >= 0)
+  if (b->vlevel >= 0 && !tree_level_abs(P.top_abs, b->vlevel, P.L))
     for (int s = 0; s < 2; ++s) b->off_vk[s] = take(BH * P.Np[b->vlevel] * d->D * 2);
   b->off_rech = CR > 64 ? take(b->max_entries * 8) : -1;
   for (int l = 0; l < P.L; ++l) {
@@ -400,10 +401,11 @@ __global__ __launch_bounds__(256) void prep_kernel(const T* __restrict__ o, cons
 // blk*16D + (d/16)*256 + (c/4)*64 + (d%16)*4 + c%4, so that the 4-node pieces
 // one MFMA operand read takes lie contiguous; the V source
 // VH[blk][c/4][d][c%4] is written back as rows VR[node][d].  One thread per (bh, node, d).
+// pairs: K~ in pair order (tree_kfrag), else in dslot's (the two differ at D = 32).
 __global__ __launch_bounds__(256) void pack_bwd_kernel(
     const uint16_t* __restrict__ kh, const uint16_t* __restrict__ kl,
     const uint16_t* __restrict__ vh, const uint16_t* __restrict__ vl, int64_t Np, int D,
-    int64_t total, uint16_t* __restrict__ kt_h, uint16_t* __restrict__ kt_l,
+    bool pairs, int64_t total, uint16_t* __restrict__ kt_h, uint16_t* __restrict__ kt_l,
     uint16_t* __restrict__ vr_h, uint16_t* __restrict__ vr_l) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= total) return;
@@ -415,7 +417,7 @@ __global__ __launch_bounds__(256) void pack_bwd_kernel(
   const int64_t tr = (bh * (Np / 16) + node / 16) * D * 16 + (dd >> 4) * 256 + (c >> 2) * 64 +
                      (dd & 15) * 4 + (c & 3);
   const int64_t vsrc = (bh * (Np / 16) + node / 16) * D * 16 + (c >> 2) * 4 * D + dd * 4 + (c & 3);
-  const int64_t ksrc = tree_kfrag(D, idx);
+  const int64_t ksrc = pairs ? tree_kfrag(D, idx) : tree_kchunk(D, idx);
   if (kt_h) kt_h[tr] = kh[ksrc];
   if (kt_l) kt_l[tr] = kl[ksrc];
   if (vr_h) vr_h[idx] = vh[vsrc];
@@ -436,7 +438,7 @@ __device__ __forceinline__ int fp16_block_exp(float amax) {
 template <int D>
 __global__ __launch_bounds__(256) void pack_kt16_kernel(const uint16_t* __restrict__ kh,
                                                         const uint16_t* __restrict__ kl, int64_t Np,
-                                                        int64_t nblk, uint16_t* __restrict__ kt,
+                                                        bool pairs, int64_t nblk, uint16_t* __restrict__ kt,
                                                         int32_t* __restrict__ kexp) {
   constexpr int PER = 16 * D / 64;
   const int lane = threadIdx.x & 63;
@@ -450,7 +452,7 @@ __global__ __launch_bounds__(256) void pack_kt16_kernel(const uint16_t* __restri
     const int o = i * 64 + lane;
     const int d = (o >> 8) * 16 + ((o & 63) >> 2);
     const int c = ((o & 255) >> 6) * 4 + (o & 3);
-    const int64_t src = tree_kfrag(D, (row0 + c) * D + d);
+    const int64_t r = (row0 + c) * D + d, src = pairs ? tree_kfrag(D, r) : tree_kchunk(D, r);
     x[i] = bf_to_f(kh[src]) + bf_to_f(kl[src]);
     amax = fmaxf(amax, fabsf(x[i]));
   }
@@ -648,8 +650,9 @@ __global__ __launch_bounds__(256) void prefix_list_kernel(int T, int Hkv, int TK
 
 // One lane per (query group, slot s): the entry of (parent p's row, t) is
 // found from the row bitmap's word prefix, and gets the rotation row
-// rho = n_c - 1 - s CR (low 16 bits, the slot s above them) and the mask of p's children that t accumulates at
-// this level (valid positions, not passed to level l-1).  A query group's
+// rho = n_c - 1 - s CR (low 16 bits, the slot s above them; abs, a level whose
+// K~ is at the angle of the node: n_c - 1) and the mask of p's children that t
+// accumulates at this level (valid positions, not passed to level l-1).  A query group's
 // TK slots are TK consecutive lanes of one wave; its next-level list is read
 // by shuffles.  emap (nullable) maps (query group, slot) to {entry, mask}.
 // Accumulate mask of p's children in one entry: the nvalid candidates (>= 1)
@@ -676,7 +679,7 @@ __global__ __launch_bounds__(256) void record_kernel(const int32_t* __restrict__
                                                      int Hkv, int TK, int64_t Pl, int64_t W,
                                                      int64_t pw, int CR, int crlg, int64_t total,
                                                      int4* __restrict__ rec, int2* __restrict__ rech,
-                                                     int4* __restrict__ emap) {
+                                                     int4* __restrict__ emap, int abs) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool in = idx < total;
   const int lane = threadIdx.x & 63;
@@ -705,7 +708,8 @@ __global__ __launch_bounds__(256) void record_kernel(const int32_t* __restrict__
   const int64_t row = (b * Hkv + h) * Pl + p;
   const int64_t wi = row * W + (t >> 5);
   const int e = rowoff[row] + wpre[wi] + __popc(bm[wi] & ((1u << (t & 31)) - 1u));
-  rec[e] = make_int4(t, (nc - 1 - (s << crlg)) | (s << 16), (int)(uint32_t)m, (int)(uint32_t)(m >> 32));
+  rec[e] = make_int4(t, (nc - 1 - (abs ? 0 : s << crlg)) | (s << 16), (int)(uint32_t)m,
+                     (int)(uint32_t)(m >> 32));
   if (rech) rech[e] = make_int2((int)(uint32_t)mh, (int)(uint32_t)(mh >> 32));
   if (emap) emap[idx] = make_int4(e, (int)(uint32_t)m, (int)(uint32_t)(m >> 32), 0);
 }
@@ -718,7 +722,7 @@ __global__ __launch_bounds__(256) void record_wide_kernel(
     const int32_t* __restrict__ par, const int32_t* __restrict__ par_next,
     const uint32_t* __restrict__ bm, const int32_t* __restrict__ wpre,
     const int32_t* __restrict__ rowoff, int T, int Hkv, int TK, int64_t Pl, int64_t W, int64_t pw,
-    int CR, int crlg, int64_t total, int4* __restrict__ rec, int2* __restrict__ rech) {
+    int CR, int crlg, int64_t total, int4* __restrict__ rec, int2* __restrict__ rech, int abs) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= total) return;
   const int p = par[idx];
@@ -760,7 +764,8 @@ __global__ __launch_bounds__(256) void record_wide_kernel(
   const int64_t row = (b * Hkv + h) * Pl + p;
   const int64_t wi = row * W + (t >> 5);
   const int e = rowoff[row] + wpre[wi] + __popc(bm[wi] & ((1u << (t & 31)) - 1u));
-  rec[e] = make_int4(t, (nc - 1 - (s << crlg)) | (s << 16), (int)(uint32_t)m, (int)(uint32_t)(m >> 32));
+  rec[e] = make_int4(t, (nc - 1 - (abs ? 0 : s << crlg)) | (s << 16), (int)(uint32_t)m,
+                     (int)(uint32_t)(m >> 32));
   if (rech) rech[e] = make_int2((int)(uint32_t)mh, (int)(uint32_t)(mh >> 32));
 }
 
@@ -784,6 +789,7 @@ struct DkvArgs {
   float scale;
   const int2* rech;  // CR 128: accumulate mask of children 64..127 (nullptr below)
   const uint16_t* dos;  // fp32 inputs: dO rows split, [B,T,H][hi D | lo D] bf16
+  int32_t abs;  // K~ is at the angle of the node, the records' rho that of the query's node
 };
 
 // One entry's inputs staged in LDS by asynchronous copies: the 16 query
@@ -1359,12 +1365,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   }
   wait_stage();
   if (!live) return;
-  // dk of the node = scale R^-1(dK~, node mod CR); write this piece's partial
+  // dk of the node = scale R^-1(dK~, node mod CR) (abs: node); write this piece's partial
   float* out = a.partial + ((pc * a.tpp + tile) * 16) * (int64_t)D * 2;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int cand = 4 * kg + r;
-    const int c = (coff + cand) & (CR - 1);
+    const int c = (a.abs ? p << crlg : 0) + ((coff + cand) & (CR - 1));
 #pragma unroll
     for (int n = 0; n < ND / 2; ++n) {
       const int i = 16 * n + u16;
@@ -1696,12 +1702,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   }
   wait_stage();
   if (!live) return;
-  // dk of the node = scale R^-1(dK~, node mod CR); write this piece's partial
+  // dk of the node = scale R^-1(dK~, node mod CR) (abs: node); write this piece's partial
   float* out = a.partial + ((pc * a.tpp + tile) * 16) * (int64_t)D * 2;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int cand = 4 * kg + r;
-    const int c = (coff + cand) & (CR - 1);
+    const int c = (a.abs ? p << crlg : 0) + ((coff + cand) & (CR - 1));
 #pragma unroll
     for (int n = 0; n < ND / 2; ++n) {
       const int i = 16 * n + u16;
@@ -1787,6 +1793,7 @@ __global__ __launch_bounds__(256) void dkv_reduce_kernel(const float* __restrict
 struct DqLevel {
   const uint16_t *kh, *kl, *kt_h, *kt_l, *vr_h, *vr_l;
   int64_t Np, pw;
+  int32_t abs;  // K~ at the angle of the node: one query frame for the level
 };
 
 struct DqArgs {
@@ -1848,7 +1855,8 @@ __device__ __forceinline__ void rot_acc(f32x4 (&x)[D / 16], const float* c, cons
 // fragment advances by R(., -CR) and the tile contributions are gathered in
 // a frame that turns with it, X <- R(X, -CR) + dq~_tile, so that
 //   sum_s R^-1(dq~_s, a - s CR) = R^-1(X, n_c-1 - (np-1) CR) = R(X, -c_t)
-// needs one table rotation per level.
+// needs one table rotation per level.  (A level whose K~ is at the angle of
+// the node has one frame, turned back by -(n_c-1).)
 template <int D, bool PREC, typename TIn, int MAXTK, int MAXPOS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 32 ? 5 : D == 256 ? 1 : 2))) void dq_kernel(const DqArgs a) {
   constexpr int KS = D / 32, ND = D / 16, HALF = D / 2;
@@ -1968,7 +1976,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 32 ? 5
         }
       }
       const int s = wide ? (tau << 4) >> crlg : tau;
-      if (s != cur_slot) {  // ascending slots, one step apart
+      if (s != cur_slot && !P.abs) {  // ascending slots, one step apart
         rot_by_fr<D>(qr, rot_m[0], rot_m[1], kg);
         rot_acc<D>(X, rot_m[0], rot_m[1], kg);
         cur_slot = s;
@@ -2040,11 +2048,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 32 ? 5
     }
     // back to the query's frame: R(X, -c_t)
     {
+      const int back = P.abs ? apos : ct;
 #pragma unroll
       for (int n = 0; n < ND / 2; ++n) {
         const int i0 = 16 * n + 4 * kg;
-        const float4 c4 = *(const float4*)(a.cosb + (int64_t)ct * HALF + i0);
-        const float4 s4 = *(const float4*)(a.sinb + (int64_t)ct * HALF + i0);
+        const float4 c4 = *(const float4*)(a.cosb + (int64_t)back * HALF + i0);
+        const float4 s4 = *(const float4*)(a.sinb + (int64_t)back * HALF + i0);
         const float cc[4] = {c4.x, c4.y, c4.z, c4.w}, ss[4] = {s4.x, s4.y, s4.z, s4.w};
         f32x4 lo4 = AC[n][lane], hi4 = AC[n + ND / 2][lane];
 #pragma unroll
@@ -2338,24 +2347,27 @@ static int backward_t(const htree_dims* d, const BwdPlan& BP, float scale, const
   const bool has_scores = !PREC && scores;  // dkv reads the stored scores
   hipLaunchKernelGGL((prep_kernel<D, T>), dim3((unsigned)((groups + 3) / 4)), dim3(256), 0, st,
                      (const T*)out, (const T*)dO, groups, d->H, G, delta, dos);
+  auto level_abs = [&](int l) { return tree_level_abs(P.top_abs, l, P.L); };
   for (int l = 0; l < P.L; ++l) {
     const int64_t total = BH * P.Np[l] * d->D;
+    // K~ at the child's angle, and its element order
+    const bool sk = level_abs(l) && P.off_sh[l] >= 0;
+    const uint16_t* ckh = (const uint16_t*)(tws + (sk ? P.off_sh[l] : P.off_kh[l]));
+    const uint16_t* ckl = (const uint16_t*)(tws + (sk ? P.off_sl[l] : P.off_kl[l]));
     // transposed K~ (fp16 / fp32 inputs) and V rows (dq_kernel)
     if (PREC || !BP.use_ds)
       hipLaunchKernelGGL(pack_bwd_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                       (const uint16_t*)(tws + P.off_kh[l]), (const uint16_t*)(tws + P.off_kl[l]),
-                       (const uint16_t*)(tws + P.off_vh[l]),
+                       ckh, ckl, (const uint16_t*)(tws + P.off_vh[l]),
                        P.off_vl[l] >= 0 ? (const uint16_t*)(tws + P.off_vl[l]) : nullptr, P.Np[l],
-                       d->D, total, PREC ? U16(BP.off_kt[0][l]) : nullptr, U16(BP.off_kt[1][l]),
+                       d->D, !sk, total, PREC ? U16(BP.off_kt[0][l]) : nullptr, U16(BP.off_kt[1][l]),
                        U16(BP.off_vr[0][l]), U16(BP.off_vr[1][l]));
     if (!PREC && BP.use_ds) {
       const int64_t nblk = BH * (P.Np[l] / 16);
       hipLaunchKernelGGL(pack_kt16_kernel<D>, dim3((unsigned)((nblk + 3) / 4)), dim3(256), 0, st,
-                         (const uint16_t*)(tws + P.off_kh[l]), (const uint16_t*)(tws + P.off_kl[l]),
-                         P.Np[l], nblk, U16(BP.off_kt[0][l]), (int32_t*)(ws + BP.off_kexp[l]));
+                         ckh, ckl, P.Np[l], !sk, nblk, U16(BP.off_kt[0][l]), (int32_t*)(ws + BP.off_kexp[l]));
     }
     // the merged level's K~ in the 64-child frame (rebuilt scores only)
-    if (l == BP.vlevel && !has_scores) {
+    if (l == BP.vlevel && !has_scores && !level_abs(l)) {
       const int64_t n = BH * P.Np[l] * (d->D / 2);
       hipLaunchKernelGGL(pack_vrot_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                          (const uint16_t*)(tws + P.off_kh[l]), (const uint16_t*)(tws + P.off_kl[l]),
@@ -2423,12 +2435,12 @@ static int backward_t(const htree_dims* d, const BwdPlan& BP, float scale, const
       hipLaunchKernelGGL(record_wide_kernel, dim3((unsigned)((ent + 255) / 256)), dim3(256), 0, s,
                          parents + l * lstride, l > 0 ? parents + (l - 1) * lstride : nullptr, bm,
                          wpre, rowoff, d->T, d->H_kv, d->top_k, Pl, BP.W, P.pw[l], CR, P.cr_log2,
-                         ent, recs, rech);
+                         ent, recs, rech, (int)level_abs(l));
     else
       hipLaunchKernelGGL(record_kernel, dim3((unsigned)((ent + 255) / 256)), dim3(256), 0, s,
                          parl, l > 0 ? parents + (l - 1) * lstride : nullptr, bm, wpre, rowoff,
                          d->T, d->H_kv, d->top_k, Pl, BP.W, P.pw[l], CRl, lgl, ent, recs, rech,
-                         BP.use_ds ? (int4*)(ws + BP.off_emap[l]) : nullptr);
+                         BP.use_ds ? (int4*)(ws + BP.off_emap[l]) : nullptr, (int)level_abs(l));
   };
   auto dkv_level = [&](int l) {
     // the level's rows: parents of vcr children (64 at the merged level)
@@ -2441,7 +2453,7 @@ static int backward_t(const htree_dims* d, const BwdPlan& BP, float scale, const
     int2* rech = BP.off_rech >= 0 ? (int2*)(ws + BP.off_rech) : nullptr;  // CR 128
     DkvArgs a;
     memset(&a, 0, sizeof(a));
-    const bool vrot = l == BP.vlevel && !has_scores;  // K~ of the 64-child frame
+    const bool vrot = l == BP.vlevel && !has_scores && !level_abs(l);  // K~ of the 64-child frame
     a.kh = vrot ? U16(BP.off_vk[0]) : (const uint16_t*)(tws + P.off_kh[l]);
     a.kl = vrot ? U16(BP.off_vk[1]) : (const uint16_t*)(tws + P.off_kl[l]);
     a.vt_h = (const uint16_t*)(tws + P.off_vh[l]);
@@ -2476,6 +2488,7 @@ static int backward_t(const htree_dims* d, const BwdPlan& BP, float scale, const
     a.tpp = tppl;
     a.max_tiles = P.max_tiles;  // the forward's tiles per level (stored-score index)
     a.scale = scale;
+    a.abs = level_abs(l);
     const int64_t waves = BP.max_pieces * tppl;
     const bool has_s = has_scores;
     if (has_s) {
@@ -2589,6 +2602,7 @@ static int backward_t(const htree_dims* d, const BwdPlan& BP, float scale, const
       a.lv[l].kt_l = U16(BP.off_kt[1][l]);
       a.lv[l].vr_h = U16(BP.off_vr[0][l]);
       a.lv[l].vr_l = U16(BP.off_vr[1][l]);
+      a.lv[l].abs = level_abs(l);
       a.lv[l].Np = P.Np[l];
       a.lv[l].pw = P.pw[l];
     }

@@ -58,13 +58,17 @@ constexpr int kSplitMaxTK = 2048;
 // Scores always use the split product (plain bf16 scores err by ~2e-2 when
 // |q||k| is large, e.g. clustered keys); VL exists for fp32/fp16 inputs only
 // (bf16 V is exact in VH).
-//   SH/SL                     D = 32: the same K~ with d in dslot's order, which
-//                               the scores that select are summed in (every
-//                               level; levels >= 1 for the wide forward).
-//                               D >= 64: KH/KL, where the two orders agree.
-//   AH/AL (wide forward)        the top level's R(K, node): its candidates are
-//                               nodes 0 .. t's, so the accumulation there meets
-//                               them with one turn of the query for the level.
+//   At the top level of the wide forward's configurations (top_abs) KH/KL hold
+//   R(K, node): the candidates there are nodes 0 .. t's, so one turn of the
+//   query meets them all.  The backward rebuilds its scores from the same
+//   arrays: from R(K, node mod CR) they would differ from the forward's by the
+//   rounding of the tables' angles (up to 3e-4 at position 8000), and P from
+//   gmax / gsum with them.
+//   SH/SL                       K~ at the child's angle with d in dslot's order,
+//                               which the scores that select are summed in.
+//                               KH/KL except at D = 32 (levels >= 1 for the wide
+//                               forward, every level for the others) and at the
+//                               wide forward's top level.
 // Rows >= N of the padding are zero.
 struct Plan {
   int L;
@@ -75,7 +79,7 @@ struct Plan {
   int64_t off_kh[HTREE_MAX_LEVELS], off_kl[HTREE_MAX_LEVELS];
   int64_t off_vh[HTREE_MAX_LEVELS], off_vl[HTREE_MAX_LEVELS];
   int64_t off_sh[HTREE_MAX_LEVELS], off_sl[HTREE_MAX_LEVELS];  // -1: none
-  int64_t off_ah, off_al;                                      // -1: none
+  bool top_abs;   // KH / KL of level L - 1 at the angle of the node
   int64_t bytes;
   int max_tiles;  // candidate tiles of 16 per level: TK * max(CR,16) / 16
   int cr_log2;
@@ -639,7 +643,7 @@ struct LevelPtrs {
   const uint16_t* kl;
   const uint16_t* vh;
   const uint16_t* vl;
-  const uint16_t* sh;  // wide forward: K~ of the scores that select
+  const uint16_t* sh;  // K~ of the scores that select (wide forward)
   const uint16_t* sl;
   int64_t N, Np, pw;
 };

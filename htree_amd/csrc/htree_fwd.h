@@ -11,7 +11,6 @@ constexpr float kNegInfSentinel = -1.0e10f;
 
 struct FwdArgs {
   LevelPtrs lv[HTREE_MAX_LEVELS];
-  const uint16_t *ah, *al;  // wide forward: the top level's R(K, node)
   const void* q;
   void* out;
   float* gmax;

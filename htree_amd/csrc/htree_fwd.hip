@@ -538,8 +538,9 @@ static int forward_impl(const htree_dims* d, float scale, const void* q, const v
   memset(&a, 0, sizeof(a));
   const char* base = (const char*)tree_ws;
   for (int l = 0; l < P.L; ++l) {
-    // the wide forward accumulates from KH / KL and selects from SH / SL
-    // (which level 0 has none of); the other forms score once, from SH / SL
+    // the wide forward accumulates from KH / KL (the top level's at the angle
+    // of the node) and selects from SH / SL, which a level that selects
+    // nothing may lack; the other forms score once, from SH / SL
     a.lv[l].kh = (const uint16_t*)(base + (wide_fwd ? P.off_kh[l] : P.off_sh[l]));
     a.lv[l].kl = (const uint16_t*)(base + (wide_fwd ? P.off_kl[l] : P.off_sl[l]));
     a.lv[l].sh = P.off_sh[l] >= 0 ? (const uint16_t*)(base + P.off_sh[l]) : nullptr;
@@ -550,8 +551,6 @@ static int forward_impl(const htree_dims* d, float scale, const void* q, const v
     a.lv[l].Np = P.Np[l];
     a.lv[l].pw = P.pw[l];
   }
-  a.ah = P.off_ah >= 0 ? (const uint16_t*)(base + P.off_ah) : nullptr;
-  a.al = P.off_al >= 0 ? (const uint16_t*)(base + P.off_al) : nullptr;
   a.q = q;
   a.out = out;
   a.gmax = gmax;

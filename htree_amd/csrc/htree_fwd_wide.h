@@ -442,8 +442,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
 #pragma unroll
       for (int n = 0; n < ND; ++n) O[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    const uint16_t* KH = (top ? a.ah : P.kh) + hrow * D;
-    const uint16_t* KL = (top ? a.al : P.kl) + hrow * D;
+    const uint16_t* KH = P.kh + hrow * D;  // (the top level's at the angle of the node)
+    const uint16_t* KL = P.kl + hrow * D;
     const uint16_t* VH = P.vh + hrow * D;
     const uint16_t* VL = PREC ? P.vl + hrow * D : nullptr;
     float qf[KS][8];

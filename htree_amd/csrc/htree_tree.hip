@@ -91,14 +91,17 @@ int make_plan(const htree_dims* d, Plan* p) {
     p->off_vl[l] = p->precise ? take(elems) : -1;
     p->off_sh[l] = p->off_kh[l];
     p->off_sl[l] = p->off_kl[l];
-    if (d->D == 32) {
-      const bool selects = l > 0 || !wide_fwd;  // (the register forward scores every level once)
-      p->off_sh[l] = selects ? take(elems) : -1;
-      p->off_sl[l] = selects ? take(elems) : -1;
+    const bool abs = wide_fwd && l == L - 1;
+    if (d->D == 32 || abs) {
+      // read by the other forms at every level (they score it once), by the
+      // wide form where it selects, and by the stored-dS backward of quads
+      // (its K~^T is at the child's angle)
+      const bool needed = l > 0 || !wide_fwd || (abs && !wide);
+      p->off_sh[l] = needed ? take(elems) : -1;
+      p->off_sl[l] = needed ? take(elems) : -1;
     }
   }
-  p->off_ah = wide_fwd ? take(BH * p->Np[L - 1] * d->D) : -1;
-  p->off_al = wide_fwd ? take(BH * p->Np[L - 1] * d->D) : -1;
+  p->top_abs = wide_fwd;
   p->bytes = off;
   // one (b, h_kv) block of a level's operand arrays is addressed through a
   // buffer resource of 32-bit range
@@ -125,11 +128,11 @@ struct BuildArgs {
   uint16_t* kl[HTREE_MAX_LEVELS];
   uint16_t* vh[HTREE_MAX_LEVELS];
   uint16_t* vl[HTREE_MAX_LEVELS];       // nullptr for bf16 inputs
-  uint16_t* sh[HTREE_MAX_LEVELS];       // D = 32: K~ in dslot's order (or nullptr)
+  uint16_t* sh[HTREE_MAX_LEVELS];       // K~ of the scores that select, where apart (or nullptr)
   uint16_t* sl[HTREE_MAX_LEVELS];
-  uint16_t *ah, *al;                    // top level's K at the angle of its node (or nullptr)
   int64_t N[HTREE_MAX_LEVELS], Np[HTREE_MAX_LEVELS], pw[HTREE_MAX_LEVELS];
   const float *cosb, *sinb;
+  bool top_abs;                         // kh / kl of level L - 1 at the angle of the node
   int64_t chunks;                       // spans per (b, h_kv)
   int Hkv, D, CR, L, lspan;             // levels 0 .. lspan-1 come from the span launch
 };
@@ -137,15 +140,13 @@ struct BuildArgs {
 // K~ of nodes nf .. nf+cnt-1 of level l: R(K, node mod CR) split into bf16
 // hi / lo; val(j, e) is element e of node nf + j.  A thread takes 4
 // consecutive RoPE pairs (i, i + D/2) of one node (8-byte stores).
-// `abs`: R(K, node) into the top level's own arrays.
+// `abs`: at the angle of the node, R(K, node).  Into kh / kl (pair order) and
+// sh / sl (dslot's), nullptr: not.
 template <typename F>
 __device__ __forceinline__ void pack_k_at(const BuildArgs& a, int l, int64_t bh, int64_t nf, int cnt,
-                                          bool abs, F val) {
+                                          bool abs, uint16_t* kh, uint16_t* kl, uint16_t* sh,
+                                          uint16_t* sl, F val) {
   const int D = a.D, HALF = D / 2, Q = D / 8;
-  uint16_t* kh = abs ? a.ah : a.kh[l];
-  uint16_t* kl = abs ? a.al : a.kl[l];
-  uint16_t* sh = abs ? nullptr : a.sh[l];
-  uint16_t* sl = a.sl[l];
   for (int it = threadIdx.x; it < cnt * Q; it += blockDim.x) {
     int j, i0;
     pack_k_item(it, D, &j, &i0);
@@ -172,11 +173,13 @@ __device__ __forceinline__ void pack_k_at(const BuildArgs& a, int l, int64_t bh,
                           r1[2 * q + 1] - __uint_as_float(h1[q] & 0xffff0000u));
     }
     const int64_t row = tree_krow(a.Np[l], D, bh, node);
-    const int64_t o0 = tree_kfrag(D, row + i0), o1 = tree_kfrag(D, row + HALF + i0);
-    *(uint2*)(kh + o0) = make_uint2(h0[0], h0[1]);
-    *(uint2*)(kh + o1) = make_uint2(h1[0], h1[1]);
-    *(uint2*)(kl + o0) = make_uint2(l0[0], l0[1]);
-    *(uint2*)(kl + o1) = make_uint2(l1[0], l1[1]);
+    if (kh) {
+      const int64_t o0 = tree_kfrag(D, row + i0), o1 = tree_kfrag(D, row + HALF + i0);
+      *(uint2*)(kh + o0) = make_uint2(h0[0], h0[1]);
+      *(uint2*)(kh + o1) = make_uint2(h1[0], h1[1]);
+      *(uint2*)(kl + o0) = make_uint2(l0[0], l0[1]);
+      *(uint2*)(kl + o1) = make_uint2(l1[0], l1[1]);
+    }
     if (sh) {
       const int64_t s0 = tree_kchunk(D, row + i0), s1 = tree_kchunk(D, row + HALF + i0);
       *(uint2*)(sh + s0) = make_uint2(h0[0], h0[1]);
@@ -189,8 +192,12 @@ __device__ __forceinline__ void pack_k_at(const BuildArgs& a, int l, int64_t bh,
 template <typename F>
 __device__ __forceinline__ void pack_k(const BuildArgs& a, int l, int64_t bh, int64_t nf, int cnt,
                                        F val) {
-  pack_k_at(a, l, bh, nf, cnt, false, val);
-  if (a.ah && l == a.L - 1) pack_k_at(a, l, bh, nf, cnt, true, val);
+  if (tree_level_abs(a.top_abs, l, a.L)) {
+    pack_k_at(a, l, bh, nf, cnt, true, a.kh[l], a.kl[l], nullptr, nullptr, val);
+    if (a.sh[l]) pack_k_at(a, l, bh, nf, cnt, false, nullptr, nullptr, a.sh[l], a.sl[l], val);
+  } else {
+    pack_k_at(a, l, bh, nf, cnt, false, a.kh[l], a.kl[l], a.sh[l], a.sl[l], val);
+  }
 }
 
 // element (d, node) of the level's V^T blocks
@@ -253,10 +260,6 @@ __device__ __forceinline__ void zero_padding(const BuildArgs& a, int64_t bh) {
         const int64_t so = tree_kchunk(D, tree_krow(a.Np[l], D, bh, node) + d);
         a.sh[l][so] = 0;
         a.sl[l][so] = 0;
-      }
-      if (a.ah && l == a.L - 1) {
-        a.ah[ko] = 0;
-        a.al[ko] = 0;
       }
       const int64_t o = vt_index(a, l, bh, node, d);
       a.vh[l][o] = 0;
@@ -415,7 +418,7 @@ static int tree_build_t(const htree_dims* d, const Plan& P, const void* k, const
     a.kl[l] = (uint16_t*)(base + P.off_kl[l]);
     a.vh[l] = (uint16_t*)(base + P.off_vh[l]);
     a.vl[l] = P.off_vl[l] >= 0 ? (uint16_t*)(base + P.off_vl[l]) : nullptr;
-    if (d->D == 32 && P.off_sh[l] >= 0) {
+    if (P.off_sh[l] >= 0 && P.off_sh[l] != P.off_kh[l]) {
       a.sh[l] = (uint16_t*)(base + P.off_sh[l]);
       a.sl[l] = (uint16_t*)(base + P.off_sl[l]);
     }
@@ -423,10 +426,7 @@ static int tree_build_t(const htree_dims* d, const Plan& P, const void* k, const
     a.Np[l] = P.Np[l];
     a.pw[l] = P.pw[l];
   }
-  if (P.off_ah >= 0) {
-    a.ah = (uint16_t*)(base + P.off_ah);
-    a.al = (uint16_t*)(base + P.off_al);
-  }
+  a.top_abs = P.top_abs;
   a.cosb = cosb;
   a.sinb = sinb;
   a.Hkv = d->H_kv;

@@ -69,6 +69,12 @@ __host__ __device__ inline int64_t tree_kfrag(int D, int64_t r) {
   return tree_kchunk(D, n * D + pair_slot32((int)(r - n * D)));
 }
 
+// Whether a level's K~ (KH / KL) is at the angle of the node, R(K, node), not
+// of the child, R(K, node mod CR).
+__host__ __device__ inline bool tree_level_abs(bool top_abs, int l, int L) {
+  return top_abs && l == L - 1;
+}
+
 // Element (d, node) of a level's V^T blocks: 16-node blocks of four 4-node
 // quads, (d, c) at (c / 4) * 4D + d * 4 + c % 4.
 __host__ __device__ inline int64_t tree_vt_index(int64_t Np, int D, int64_t bh, int64_t node,

@@ -48,3 +48,42 @@ def test_max_is_a_score(B, T, H, Hkv, D, CR, TK, MTN, dtype):
                                               10000.0)
     torch.cuda.synchronize()
     assert torch.equal(tr["layers"][0].layer_max[:, 0].cpu().double(), want)
+
+
+CONSISTENT = [
+    # T, H, Hkv, D, CR, TK, MTN, dtype
+    (8000, 4, 1, 32, 16, 512, 8192, torch.float32),   # wide form, one level
+    (9001, 8, 1, 32, 16, 512, 8192, torch.float32),   # two levels
+    (8000, 4, 1, 32, 16, 512, 8192, torch.bfloat16),  # two entries per dkv tile
+    (8000, 4, 1, 128, 16, 512, 8192, torch.float32),
+    (3000, 16, 1, 32, 64, 64, 4096, torch.float32),   # top_k 64 in four tiles each
+    (3000, 8, 1, 64, 4, 512, 2048, torch.bfloat16),   # slots of four
+    (4000, 34, 1, 32, 16, 16, 256, torch.float32),    # a quad, the merged top level
+    (2000, 50, 1, 64, 16, 16, 128, torch.bfloat16),   # a quad, stored dS
+    (8000, 8, 1, 64, 32, 32, 256, torch.float32),     # streaming form
+    (4000, 8, 1, 64, 16, 16, 256, torch.float32),     # register form
+]
+
+
+@pytest.mark.parametrize("T,H,Hkv,D,CR,TK,MTN,dtype", CONSISTENT)
+def test_probabilities_of_the_backward_sum_to_one(T, H, Hkv, D, CR, TK, MTN, dtype):
+    """dO = e_i at D chosen queries (one head and one element i each) makes the
+    sum of dv[..., i] over all tokens that query's sum of P as the backward
+    rebuilds it.  Its scores and the forward's differ in the residuals of the
+    queries' and keys' bf16 splits (at most 2^-17 of an element each, and
+    2^-18 / sqrt(3) of it on average): with |q| of 2 sqrt(D), |k| of sqrt(D) and the
+    scale 1 / sqrt(D) about 2^-17 = 7.6e-6 a score.  The bar is three times
+    that.  (K~ at other angles in the two passes: 6e-5 in the first case.)"""
+    g = torch.Generator().manual_seed(5)
+    q = (2 * torch.randn(1, T, H, D, generator=g)).to(dtype).to(DEV)
+    k = torch.randn(1, T, Hkv, D, generator=g).to(dtype).to(DEV)
+    v = torch.randn(1, T, Hkv, D, generator=g).to(dtype).to(DEV)
+    dO = torch.zeros_like(q)
+    i = torch.arange(D)
+    dO[0, torch.linspace(T // 2, T - 1, D).long(), i % H, i] = 1
+    out, ctx = htree_amd.htree_forward(q, k, v, CR, MTN, TK, _save_for_backward=True)
+    dv = htree_amd.htree_backward(dO, q, out, ctx)[2]
+    torch.cuda.synchronize()
+    off = (dv.double().sum((0, 1, 2)) - 1).abs().max().item()
+    print(off, flush=True)
+    assert off <= 2.3e-5

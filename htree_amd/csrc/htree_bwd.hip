@@ -401,7 +401,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const T* __restrict__ o, cons
 // blk*16D + (d/16)*256 + (c/4)*64 + (d%16)*4 + c%4, so that the 4-node pieces
 // one MFMA operand read takes lie contiguous; the V source
 // VH[blk][c/4][d][c%4] is written back as rows VR[node][d].  One thread per (bh, node, d).
-// pairs: K~ in pair order (tree_kfrag), else in dslot's (the two differ at D = 32).
+// pairs: K~ in pair order (tree_kindex).
 __global__ __launch_bounds__(256) void pack_bwd_kernel(
     const uint16_t* __restrict__ kh, const uint16_t* __restrict__ kl,
     const uint16_t* __restrict__ vh, const uint16_t* __restrict__ vl, int64_t Np, int D,
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(256) void pack_bwd_kernel(
   const int64_t tr = (bh * (Np / 16) + node / 16) * D * 16 + (dd >> 4) * 256 + (c >> 2) * 64 +
                      (dd & 15) * 4 + (c & 3);
   const int64_t vsrc = (bh * (Np / 16) + node / 16) * D * 16 + (c >> 2) * 4 * D + dd * 4 + (c & 3);
-  const int64_t ksrc = pairs ? tree_kfrag(D, idx) : tree_kchunk(D, idx);
+  const int64_t ksrc = tree_kindex(D, pairs, idx);
   if (kt_h) kt_h[tr] = kh[ksrc];
   if (kt_l) kt_l[tr] = kl[ksrc];
   if (vr_h) vr_h[idx] = vh[vsrc];
@@ -452,7 +452,7 @@ __global__ __launch_bounds__(256) void pack_kt16_kernel(const uint16_t* __restri
     const int o = i * 64 + lane;
     const int d = (o >> 8) * 16 + ((o & 63) >> 2);
     const int c = ((o & 255) >> 6) * 4 + (o & 3);
-    const int64_t r = (row0 + c) * D + d, src = pairs ? tree_kfrag(D, r) : tree_kchunk(D, r);
+    const int64_t src = tree_kindex(D, pairs, (row0 + c) * D + d);
     x[i] = bf_to_f(kh[src]) + bf_to_f(kl[src]);
     amax = fmaxf(amax, fabsf(x[i]));
   }
@@ -471,8 +471,8 @@ __global__ __launch_bounds__(256) void pack_kt16_kernel(const uint16_t* __restri
 // is exact in fp32; the turned value is split again into hi + lo.  One
 // thread per (bh, node, RoPE pair i); padding rows stay zero.
 __global__ __launch_bounds__(256) void pack_vrot_kernel(
-    const uint16_t* __restrict__ kh, const uint16_t* __restrict__ kl, int64_t Np, int D, int crlg,
-    int vmask, const float* __restrict__ cosb, const float* __restrict__ sinb, int64_t total,
+    const uint16_t* __restrict__ kh, const uint16_t* __restrict__ kl, int64_t Np, int D, bool pairs,
+    int crlg, int vmask, const float* __restrict__ cosb, const float* __restrict__ sinb, int64_t total,
     uint16_t* __restrict__ oh, uint16_t* __restrict__ ol) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= total) return;
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(256) void pack_vrot_kernel(
   const int64_t r = idx / half;  // bh * Np + node
   const int64_t node = r % Np;
   const int64_t a = ((node >> crlg) & vmask) << crlg;  // table row of the added angle
-  const int64_t e0 = tree_kfrag(D, r * D + i), e1 = tree_kfrag(D, r * D + i + half);
+  const int64_t e0 = tree_kindex(D, pairs, r * D + i), e1 = tree_kindex(D, pairs, r * D + i + half);
   const float x0 = bf_to_f(kh[e0]) + bf_to_f(kl[e0]);
   const float x1 = bf_to_f(kh[e1]) + bf_to_f(kl[e1]);
   const float c = cosb[a * half + i], sn = sinb[a * half + i];
@@ -789,6 +789,7 @@ struct DkvArgs {
   float scale;
   const int2* rech;  // CR 128: accumulate mask of children 64..127 (nullptr below)
   const uint16_t* dos;  // fp32 inputs: dO rows split, [B,T,H][hi D | lo D] bf16
+  int32_t pairs;  // K~ in pair order (tree_kfrag)
   int32_t abs;  // K~ is at the angle of the node, the records' rho that of the query's node
 };
 
@@ -1106,8 +1107,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   bf16x8 kh[KS], kl[KS], vh[KS], vl[KS];
   {
     if (!HAS_S) {  // K~ only rebuilds the scores
-      load_kfrag<D>(a.kh + bh * a.Np * D, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kh);
-      load_kfrag<D>(a.kl + bh * a.Np * D, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kl);
+      load_kpairs<D>(a.kh + bh * a.Np * D, a.pairs, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kh);
+      load_kpairs<D>(a.kl + bh * a.Np * D, a.pairs, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kl);
     }
     const int64_t vnode = (live ? node0 : 0) + (u16 < CRU ? u16 : 0);
     load_frag_vt<D>(a.vt_h, bh, a.Np, vnode, kg, vh);
@@ -1512,8 +1513,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   };
   bf16x8 kh[KS], kl[KS], vh[KS];
   {
-    load_kfrag<D>(a.kh + bh * a.Np * D, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kh);
-    load_kfrag<D>(a.kl + bh * a.Np * D, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kl);
+    load_kpairs<D>(a.kh + bh * a.Np * D, a.pairs, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kh);
+    load_kpairs<D>(a.kl + bh * a.Np * D, a.pairs, live ? node0 : 0, u16 < CRU ? u16 : 0, kg, kl);
     load_frag_vt<D>(a.vt_h, bh, a.Np, (live ? node0 : 0) + (u16 < CRU ? u16 : 0), kg, vh);
   }
   f32x4 dv[ND], dk[ND];
@@ -1806,6 +1807,7 @@ struct DqArgs {
   void* dq;
   int32_t B, T, H, Hkv, G, CR, crlg, TK, L;
   int32_t gdt;  // enum htree_dtype of dq
+  int32_t pairs;  // K~ in pair order (tree_kfrag)
   float scale;
 };
 
@@ -1947,8 +1949,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 32 ? 5
       const int posk = wide ? (tau << 4) + u16 : (tau << crlg) + u16;
       const bool cvk = u16 < CRU && posk < nc;
       const int node0 = node0_of(tau), c = cvk ? u16 : 0;
-      load_kfrag<D>(P.kh + hrow * D, node0, c, kg, kh);
-      load_kfrag<D>(P.kl + hrow * D, node0, c, kg, kl);
+      load_kpairs<D>(P.kh + hrow * D, a.pairs, node0, c, kg, kh);
+      load_kpairs<D>(P.kl + hrow * D, a.pairs, node0, c, kg, kl);
     };
     // query frame of slot 0: angle apos
     float qr[KS][8];
@@ -2351,7 +2353,7 @@ static int backward_t(const htree_dims* d, const BwdPlan& BP, float scale, const
   for (int l = 0; l < P.L; ++l) {
     const int64_t total = BH * P.Np[l] * d->D;
     // K~ at the child's angle, and its element order
-    const bool sk = level_abs(l) && P.off_sh[l] >= 0;
+    const bool sk = level_abs(l) && P.off_sh[l] >= 0, prs = P.pairs && !sk;
     const uint16_t* ckh = (const uint16_t*)(tws + (sk ? P.off_sh[l] : P.off_kh[l]));
     const uint16_t* ckl = (const uint16_t*)(tws + (sk ? P.off_sl[l] : P.off_kl[l]));
     // transposed K~ (fp16 / fp32 inputs) and V rows (dq_kernel)
@@ -2359,19 +2361,19 @@ static int backward_t(const htree_dims* d, const BwdPlan& BP, float scale, const
       hipLaunchKernelGGL(pack_bwd_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
                        ckh, ckl, (const uint16_t*)(tws + P.off_vh[l]),
                        P.off_vl[l] >= 0 ? (const uint16_t*)(tws + P.off_vl[l]) : nullptr, P.Np[l],
-                       d->D, !sk, total, PREC ? U16(BP.off_kt[0][l]) : nullptr, U16(BP.off_kt[1][l]),
+                       d->D, prs, total, PREC ? U16(BP.off_kt[0][l]) : nullptr, U16(BP.off_kt[1][l]),
                        U16(BP.off_vr[0][l]), U16(BP.off_vr[1][l]));
     if (!PREC && BP.use_ds) {
       const int64_t nblk = BH * (P.Np[l] / 16);
       hipLaunchKernelGGL(pack_kt16_kernel<D>, dim3((unsigned)((nblk + 3) / 4)), dim3(256), 0, st,
-                         ckh, ckl, P.Np[l], !sk, nblk, U16(BP.off_kt[0][l]), (int32_t*)(ws + BP.off_kexp[l]));
+                         ckh, ckl, P.Np[l], prs, nblk, U16(BP.off_kt[0][l]), (int32_t*)(ws + BP.off_kexp[l]));
     }
     // the merged level's K~ in the 64-child frame (rebuilt scores only)
     if (l == BP.vlevel && !has_scores && !level_abs(l)) {
       const int64_t n = BH * P.Np[l] * (d->D / 2);
       hipLaunchKernelGGL(pack_vrot_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                          (const uint16_t*)(tws + P.off_kh[l]), (const uint16_t*)(tws + P.off_kl[l]),
-                         P.Np[l], d->D, P.cr_log2, BP.vm[l] - 1, cosb, sinb, n, U16(BP.off_vk[0]),
+                         P.Np[l], d->D, prs, P.cr_log2, BP.vm[l] - 1, cosb, sinb, n, U16(BP.off_vk[0]),
                          U16(BP.off_vk[1]));
     }
   }
@@ -2488,6 +2490,7 @@ static int backward_t(const htree_dims* d, const BwdPlan& BP, float scale, const
     a.tpp = tppl;
     a.max_tiles = P.max_tiles;  // the forward's tiles per level (stored-score index)
     a.scale = scale;
+    a.pairs = P.pairs;
     a.abs = level_abs(l);
     const int64_t waves = BP.max_pieces * tppl;
     const bool has_s = has_scores;
@@ -2625,6 +2628,7 @@ static int backward_t(const htree_dims* d, const BwdPlan& BP, float scale, const
     a.crlg = P.cr_log2;
     a.TK = d->top_k;
     a.L = Ltop + 1;
+    a.pairs = P.pairs;
     a.scale = scale;
     // LDS sized for the lists and positions: one-wave-per-group forwards
     // (64, 64 tiles), the reference's default regime (512, 8192), beyond

@@ -45,7 +45,7 @@ constexpr int kSplitMaxTK = 2048;
 //                               R(K_l[node], node mod CR), in blocks of 16
 //                               nodes laid out as the MFMA operand reads them
 //                               (element (c, d) at (d/8)*128 + c*8 + d%8;
-//                               D = 32: d in pair order, tree_kfrag):
+//                               D = 32 with pairs: d in pair order, tree_kfrag):
 //                               an operand load of a tile is 1 KB in a row.
 //                               With rows of 2 D bytes its lanes fell on 16
 //                               lines in 16-byte pieces, and the forwards were
@@ -66,9 +66,12 @@ constexpr int kSplitMaxTK = 2048;
 //   gmax / gsum with them.
 //   SH/SL                       K~ at the child's angle with d in dslot's order,
 //                               which the scores that select are summed in.
-//                               KH/KL except at D = 32 (levels >= 1 for the wide
-//                               forward, every level for the others) and at the
-//                               wide forward's top level.
+//                               KH/KL but for the wide forward: there apart from
+//                               them at the top level, and at D = 32, where KH/KL
+//                               are in pair order, at every level that selects.
+//                               (For the other forms a second copy at D = 32
+//                               would be 1.5 to 1.67 times the tree; their
+//                               backward picks the pairs from dslot's order.)
 // Rows >= N of the padding are zero.
 struct Plan {
   int L;
@@ -79,6 +82,7 @@ struct Plan {
   int64_t off_kh[HTREE_MAX_LEVELS], off_kl[HTREE_MAX_LEVELS];
   int64_t off_vh[HTREE_MAX_LEVELS], off_vl[HTREE_MAX_LEVELS];
   int64_t off_sh[HTREE_MAX_LEVELS], off_sl[HTREE_MAX_LEVELS];  // -1: none
+  bool pairs;     // KH / KL in pair order (tree_kfrag; differs from dslot's at D = 32)
   bool top_abs;   // KH / KL of level L - 1 at the angle of the node
   int64_t bytes;
   int max_tiles;  // candidate tiles of 16 per level: TK * max(CR,16) / 16
@@ -657,6 +661,21 @@ __device__ __forceinline__ void load_kfrag(const uint16_t* __restrict__ base, in
   const uint16_t* p = base + (int64_t)(node0 & ~15) * D + (((node0 & 15) + c) * 8 + kg * 128);
 #pragma unroll
   for (int m = 0; m < D / 32; ++m) f[m] = *(const bf16x8*)(p + m * 512);
+}
+
+// The same in pair order from either order of the blocks: D = 32 in dslot's
+// order holds pairs 4 kg .. 4 kg + 3 in two 8-byte pieces.
+template <int D>
+__device__ __forceinline__ void load_kpairs(const uint16_t* __restrict__ base, bool pairs, int node0,
+                                            int c, int kg, bf16x8 (&f)[D / 32]) {
+  if (D != 32 || pairs) {
+    load_kfrag<D>(base, node0, c, kg, f);
+  } else {
+    const uint16_t* p = base + (int64_t)(node0 & ~15) * D +
+                        (((node0 & 15) + c) * 8 + (kg >> 1) * 128 + (kg & 1) * 4);
+    const uint2 lo = *(const uint2*)p, hi = *(const uint2*)(p + 256);
+    f[0] = __builtin_bit_cast(bf16x8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+  }
 }
 
 // exp(x) for x <= 0 (x = -inf gives 0) including subnormal results, which

@@ -540,9 +540,9 @@ static int forward_impl(const htree_dims* d, float scale, const void* q, const v
   for (int l = 0; l < P.L; ++l) {
     // the wide forward accumulates from KH / KL (the top level's at the angle
     // of the node) and selects from SH / SL, which a level that selects
-    // nothing may lack; the other forms score once, from SH / SL
-    a.lv[l].kh = (const uint16_t*)(base + (wide_fwd ? P.off_kh[l] : P.off_sh[l]));
-    a.lv[l].kl = (const uint16_t*)(base + (wide_fwd ? P.off_kl[l] : P.off_sl[l]));
+    // nothing may lack; for the other forms the two are one
+    a.lv[l].kh = (const uint16_t*)(base + (P.off_kh[l]));
+    a.lv[l].kl = (const uint16_t*)(base + (P.off_kl[l]));
     a.lv[l].sh = P.off_sh[l] >= 0 ? (const uint16_t*)(base + P.off_sh[l]) : nullptr;
     a.lv[l].sl = P.off_sl[l] >= 0 ? (const uint16_t*)(base + P.off_sl[l]) : nullptr;
     a.lv[l].vh = (const uint16_t*)(base + P.off_vh[l]);

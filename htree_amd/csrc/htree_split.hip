@@ -568,8 +568,8 @@ int split_forward(const htree_dims* d, const Plan& P, float scale, const void* q
   memset(&a, 0, sizeof(a));
   const char* base = (const char*)tree_ws;
   for (int l = 0; l < P.L; ++l) {
-    a.lv[l].kh = (const uint16_t*)(base + P.off_sh[l]);
-    a.lv[l].kl = (const uint16_t*)(base + P.off_sl[l]);
+    a.lv[l].kh = (const uint16_t*)(base + P.off_kh[l]);
+    a.lv[l].kl = (const uint16_t*)(base + P.off_kl[l]);
     a.lv[l].vh = (const uint16_t*)(base + P.off_vh[l]);
     a.lv[l].vl = P.off_vl[l] >= 0 ? (const uint16_t*)(base + P.off_vl[l]) : nullptr;
     a.lv[l].N = P.N[l];

@@ -92,15 +92,15 @@ int make_plan(const htree_dims* d, Plan* p) {
     p->off_sh[l] = p->off_kh[l];
     p->off_sl[l] = p->off_kl[l];
     const bool abs = wide_fwd && l == L - 1;
-    if (d->D == 32 || abs) {
-      // read by the other forms at every level (they score it once), by the
-      // wide form where it selects, and by the stored-dS backward of quads
+    if (wide_fwd && (d->D == 32 || abs)) {
+      // read where the level selects, and by the stored-dS backward of quads
       // (its K~^T is at the child's angle)
-      const bool needed = l > 0 || !wide_fwd || (abs && !wide);
+      const bool needed = l > 0 || (abs && !wide);
       p->off_sh[l] = needed ? take(elems) : -1;
       p->off_sl[l] = needed ? take(elems) : -1;
     }
   }
+  p->pairs = wide_fwd || d->D != 32;
   p->top_abs = wide_fwd;
   p->bytes = off;
   // one (b, h_kv) block of a level's operand arrays is addressed through a
@@ -132,6 +132,7 @@ struct BuildArgs {
   uint16_t* sl[HTREE_MAX_LEVELS];
   int64_t N[HTREE_MAX_LEVELS], Np[HTREE_MAX_LEVELS], pw[HTREE_MAX_LEVELS];
   const float *cosb, *sinb;
+  bool pairs;                           // kh / kl in pair order (else dslot's: D = 32)
   bool top_abs;                         // kh / kl of level L - 1 at the angle of the node
   int64_t chunks;                       // spans per (b, h_kv)
   int Hkv, D, CR, L, lspan;             // levels 0 .. lspan-1 come from the span launch
@@ -140,8 +141,8 @@ struct BuildArgs {
 // K~ of nodes nf .. nf+cnt-1 of level l: R(K, node mod CR) split into bf16
 // hi / lo; val(j, e) is element e of node nf + j.  A thread takes 4
 // consecutive RoPE pairs (i, i + D/2) of one node (8-byte stores).
-// `abs`: at the angle of the node, R(K, node).  Into kh / kl (pair order) and
-// sh / sl (dslot's), nullptr: not.
+// `abs`: at the angle of the node, R(K, node).  Into kh / kl and sh / sl
+// (dslot's order), nullptr: not.
 template <typename F>
 __device__ __forceinline__ void pack_k_at(const BuildArgs& a, int l, int64_t bh, int64_t nf, int cnt,
                                           bool abs, uint16_t* kh, uint16_t* kl, uint16_t* sh,
@@ -174,7 +175,7 @@ __device__ __forceinline__ void pack_k_at(const BuildArgs& a, int l, int64_t bh,
     }
     const int64_t row = tree_krow(a.Np[l], D, bh, node);
     if (kh) {
-      const int64_t o0 = tree_kfrag(D, row + i0), o1 = tree_kfrag(D, row + HALF + i0);
+      const int64_t o0 = tree_kindex(D, a.pairs, row + i0), o1 = tree_kindex(D, a.pairs, row + HALF + i0);
       *(uint2*)(kh + o0) = make_uint2(h0[0], h0[1]);
       *(uint2*)(kh + o1) = make_uint2(h1[0], h1[1]);
       *(uint2*)(kl + o0) = make_uint2(l0[0], l0[1]);
@@ -253,7 +254,7 @@ __device__ __forceinline__ void zero_padding(const BuildArgs& a, int64_t bh) {
     for (int it = threadIdx.x; it < np * D; it += blockDim.x) {
       const int j = it / D, d = it - j * D;
       const int64_t node = a.N[l] + j;
-      const int64_t ko = tree_kfrag(D, tree_krow(a.Np[l], D, bh, node) + d);
+      const int64_t ko = tree_kindex(D, a.pairs, tree_krow(a.Np[l], D, bh, node) + d);
       a.kh[l][ko] = 0;
       a.kl[l][ko] = 0;
       if (a.sh[l]) {
@@ -426,6 +427,7 @@ static int tree_build_t(const htree_dims* d, const Plan& P, const void* k, const
     a.Np[l] = P.Np[l];
     a.pw[l] = P.pw[l];
   }
+  a.pairs = P.pairs;
   a.top_abs = P.top_abs;
   a.cosb = cosb;
   a.sinb = sinb;

@@ -69,6 +69,11 @@ __host__ __device__ inline int64_t tree_kfrag(int D, int64_t r) {
   return tree_kchunk(D, n * D + pair_slot32((int)(r - n * D)));
 }
 
+// KH / KL in pair order or in dslot's (the two differ at D = 32).
+__host__ __device__ inline int64_t tree_kindex(int D, bool pairs, int64_t r) {
+  return pairs ? tree_kfrag(D, r) : tree_kchunk(D, r);
+}
+
 // Whether a level's K~ (KH / KL) is at the angle of the node, R(K, node), not
 // of the child, R(K, node mod CR).
 __host__ __device__ inline bool tree_level_abs(bool top_abs, int l, int L) {

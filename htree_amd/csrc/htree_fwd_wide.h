@@ -72,6 +72,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
   // (D = 64 with the keys too: 300 spills, 16.7 against 17.0 ms).
   constexpr bool PIPE = D == 32;
   constexpr bool VPIPE = D <= 64;
+  // P in bf16 hi + lo.  bf16 inputs at D <= 64 too: a batch's one softmax step
+  // leaves fewer P that are exactly 1 than a step per tile (output error against
+  // float64, D 32, T 4000: 1.96e-3 with a step per tile, 2.01e-3, and 1.62e-3
+  // with P split).  A step per tile where some head's max rises, which more
+  // than half of the batches see, cost more: T 8000, 64/4 heads, D 64 3.01 ->
+  // 3.43 ms, P split 3.29.
+  constexpr bool PSPLIT = PREC || UA > 1;
   static_assert(NH == 1 || NH == 2 || NH == 4, "parts of a block");
   // waves per part, threads
   constexpr int NW = kWideWaves / NH, NT = 64 * kWideWaves;
@@ -606,7 +613,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
           const uint32_t h01 = cvt_pk_bf16(p[0], p[1]), h23 = cvt_pk_bf16(p[2], p[3]);
           const s16x4 ph = __builtin_bit_cast(s16x4, make_uint2(h01, h23));
           s16x4 pl = ph;
-          if (PREC) {
+          if (PSPLIT) {
             const uint32_t l01 = cvt_pk_bf16(p[0] - __uint_as_float(h01 << 16),
                                              p[1] - __uint_as_float(h01 & 0xffff0000u));
             const uint32_t l23 = cvt_pk_bf16(p[2] - __uint_as_float(h23 << 16),
@@ -620,13 +627,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
             const s16x4 v1 = __builtin_bit_cast(s16x4, make_uint2(w.z, w.w));
             O[2 * i] = mma16(v0, ph, O[2 * i]);
             O[2 * i + 1] = mma16(v1, ph, O[2 * i + 1]);
+            if (PSPLIT) {
+              O[2 * i] = mma16(v0, pl, O[2 * i]);
+              O[2 * i + 1] = mma16(v1, pl, O[2 * i + 1]);
+            }
             if (PREC) {
               const uint4 wl = vl[j][i];
               const s16x4 l0 = __builtin_bit_cast(s16x4, make_uint2(wl.x, wl.y));
               const s16x4 l1 = __builtin_bit_cast(s16x4, make_uint2(wl.z, wl.w));
-              O[2 * i] = mma16(v0, pl, O[2 * i]);
               O[2 * i] = mma16(l0, ph, O[2 * i]);
-              O[2 * i + 1] = mma16(v1, pl, O[2 * i + 1]);
               O[2 * i + 1] = mma16(l1, ph, O[2 * i + 1]);
             }
           }

@@ -87,3 +87,20 @@ def test_probabilities_of_the_backward_sum_to_one(T, H, Hkv, D, CR, TK, MTN, dty
     off = (dv.double().sum((0, 1, 2)) - 1).abs().max().item()
     print(off, flush=True)
     assert off <= 2.3e-5
+
+
+@pytest.mark.parametrize("H,D,TK,MTN", [(8, 32, 128, 2048), (16, 64, 128, 128), (64, 64, 16, 128)])
+def test_wide_probabilities_beyond_bf16(H, D, TK, MTN):
+    """The wide form at D <= 64 multiplies V by P in bf16 hi + lo for bf16 inputs
+    too: with V = 1 a level's output is its sum of P.  The split leaves 2^-18
+    of a P, the fp32 sums of up to 1500 terms a few 2^-24 each; P rounded to
+    bf16 (2^-9) is off by 1e-3 where few candidates matter."""
+    g = torch.Generator().manual_seed(9)
+    q = torch.randn(1, 1500, H, D, generator=g).to(torch.bfloat16).to(DEV)
+    k = torch.randn(1, 1500, 1, D, generator=g).to(torch.bfloat16).to(DEV)
+    _, tr = htree_amd.run_parallel_with_trace(q, k, torch.ones_like(k), 16, MTN, TK, None, 10000.0)
+    torch.cuda.synchronize()
+    for lt in tr["layers"].values():
+        some = lt.layer_sum > 0
+        ratio = lt.layer_output[some].double() / lt.layer_sum[some].double()[:, None]
+        assert (ratio - 1).abs().max().item() <= 2 ** -15 if some.any() else True

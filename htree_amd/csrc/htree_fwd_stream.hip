@@ -230,10 +230,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     float qr[KS][8];
     bf16x8 qh[KS], ql[KS];
     int cur_slot = 0;
-    auto frame_start = [&]() {
+    auto frame_start = [&](const TIn* p, bool live) {
       // (read again at each pass: held, its registers spill at D = 128)
       QFrag<D, TIn, false> qin;
-      qin.load(qp, kg, gv || a.gpad == 0);
+      qin.load(p, kg, live);
       qin.get(qr, a.scale);
       rot_by<D>(qr, a.cosb + (int64_t)apos * HALF, a.sinb + (int64_t)apos * HALF, kg);
       if (ONCE) to_bf_split<D>(qr, qh, ql);
@@ -252,17 +252,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     if (upper) {
       float Mrun = -INFINITY;
       float hm[4];  // 1 for heads 4kg + r of the selection (formed per level)
-      f32x4 hinit;
       {
         int kq = kg;
         asm volatile("" : "+v"(kq));
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          hm[r] = 4 * kq + r < Gs ? 1.f : 0.f;
-          hinit[r] = 4 * kq + r < Gs || a.gpad == 0 ? 0.f : -INFINITY;
-        }
+        for (int r = 0; r < 4; ++r) hm[r] = 4 * kq + r < Gs ? 1.f : 0.f;
       }
-      frame_start();
+      // (rows past the heads of the selection repeat them here: no row's
+      // score is out of the range of the others)
+      frame_start(a.gpad == 0 ? qp : qp + (u16 < Gs ? 0 : u16 % Gs - (gv ? u16 : 0)) * D, true);
       issue(0, false);
       for (int tau = 0; tau < nt; ++tau) {
         frame_to(slot_of(tau));
@@ -271,21 +269,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
         kread(tau, kh, kl);
         reads_done();
         if (tau + 1 < nt) issue(tau + 1, false);
-        f32x4 S = hinit;
+        f32x4 S = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int m = 0; m < KS; ++m) {
           S = mma32(qh[m], kh[m], S);
           S = mma32(qh[m], kl[m], S);
           S = mma32(ql[m], kh[m], S);
         }
-        // S[r] = score[g = 4kg + r][candidate u16]
+        // S[r] = score[g = 4kg + r][candidate u16].  A column that is no
+        // candidate is kept out of the max and its sum not read; its scores
+        // (of some node of the tree) stay as they are, so that the subnormal
+        // test below sees no -inf
+        float tm = fmaxf(fmaxf(S[0], S[1]), fmaxf(S[2], S[3]));
         if (!wide || tau == nt - 1) {
           const int pos = wide ? (tau << 4) + u16 : (tau << crlg) + u16;
-          const bool cv = u16 < CRU && pos < nc;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) S[r] = cv ? S[r] : -INFINITY;
+          tm = u16 < CRU && pos < nc ? tm : -INFINITY;
         }
-        Mrun = fmaxf(Mrun, wave_max(fmaxf(fmaxf(S[0], S[1]), fmaxf(S[2], S[3]))));
+        Mrun = fmaxf(Mrun, wave_max(tm));
 #pragma unroll
         for (int r = 0; r < 4; ++r) S[r] = (S[r] - Mrun) * kLog2e;
         // subnormal results (exp_sel), one wave test for the tile
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
 #pragma unroll
       for (int n = 0; n < ND; ++n) O[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    frame_start();
+    frame_start(qp, gv || a.gpad == 0);
     issue(0, true);
     for (int tau = 0; tau < nt; ++tau) {
       frame_to(slot_of(tau));

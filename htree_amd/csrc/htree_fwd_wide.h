@@ -239,28 +239,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
       // ---- importance of every candidate (relative to the wave's running max)
       const uint16_t* KH = P.sh + hrow * D;
       const uint16_t* KL = P.sl + hrow * D;
+      // rows past the heads of the selection repeat them: no row's score is
+      // out of the range of the others
+      const TIn* qs = (const TIn*)a.q +
+                      (((int64_t)b * a.T + t) * a.H + h * G + (u16 < Gs ? u16 : u16 % Gs)) * D;
       float qf[KS][8], qo[8];
 #pragma unroll
       for (int m = 0; m < KS; ++m) {
-        Io<TIn>::ld8(qp + dslot<D>(kg, m), qf[m]);
+        Io<TIn>::ld8(qs + dslot<D>(kg, m), qf[m]);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) qf[m][e] = zero_row ? 0.f : qf[m][e] * a.scale;
+        for (int e = 0; e < 8; ++e) qf[m][e] *= a.scale;
       }
       if constexpr (D == 32) {  // the other halves of the lane's pairs, signed for the turn
-        Io<TIn>::ld8(qp + (dslot<D>(kg, 0) ^ 16), qo);
+        Io<TIn>::ld8(qs + (dslot<D>(kg, 0) ^ 16), qo);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          qo[e] = zero_row ? 0.f : qo[e] * a.scale;
-          qo[e] = kg < 2 ? -qo[e] : qo[e];
-        }
+        for (int e = 0; e < 8; ++e) qo[e] *= kg < 2 ? -a.scale : a.scale;
       }
       float hm[4];  // 1 for heads of the selection
-      f32x4 hinit;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        hm[r] = 4 * kg + r < Gs ? 1.f : 0.f;
-        hinit[r] = 4 * kg + r < Gs || a.gpad == 0 ? 0.f : -INFINITY;
-      }
+      for (int r = 0; r < 4; ++r) hm[r] = 4 * kg + r < Gs ? 1.f : 0.f;
       float Mrun = -INFINITY;
       auto tile_at = [&](int i0, int j) { return i0 + NW * j < nt ? i0 + NW * j : nt - 1; };
       auto row_at = [&](int i0, int j) { return apos - (slot_of(tile_at(i0, j)) << crlg); };
@@ -317,7 +314,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
             load_k(KH, node0, kh[j]);
             load_k(KL, node0, kl[j]);
           }
-          S[j] = hinit;
+          S[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int m = 0; m < KS; ++m) {
             S[j] = mma32(qh[m], kh[j][m], S[j]);
@@ -327,19 +324,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
           if (!PIPE) __builtin_amdgcn_sched_barrier(0);  // one tile's keys in registers
         }
         if (PIPE) keys(i0 + U * NW < nt ? i0 + U * NW : i0);
-        // S[j][r] = score[g = 4kg + r][candidate u16 of tile i0 + NW j]
+        // S[j][r] = score[g = 4kg + r][candidate u16 of tile i0 + NW j].  A
+        // column that is no candidate is kept out of the max and its sum not
+        // stored; its scores (of some node of the tree) stay as they are, so
+        // that the subnormal test below sees no -inf
+        float tm[U], M[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) tm[j] = fmaxf(fmaxf(S[j][0], S[j][1]), fmaxf(S[j][2], S[j][3]));
         if (!wide || i0 + NW * (U - 1) >= nt - 1) {
 #pragma unroll
           for (int j = 0; j < U; ++j) {
             const int tau = i0 + NW * j;
             const bool cv = tau < nt && u16 < CRU && (tau << lgt) + u16 < nc;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) S[j][r] = cv ? S[j][r] : -INFINITY;
+            tm[j] = cv ? tm[j] : -INFINITY;
           }
         }
-        float tm[U], M[U];
-#pragma unroll
-        for (int j = 0; j < U; ++j) tm[j] = fmaxf(fmaxf(S[j][0], S[j][1]), fmaxf(S[j][2], S[j][3]));
         const float tmx = row_max16(groups4(tm[0], tm[1], tm[2], tm[3], [](float x, float y) { return fmaxf(x, y); }));
 #pragma unroll
         for (int j = 0; j < U; ++j) {

@@ -473,6 +473,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
       constexpr int FORM = decltype(form)::value;
       const bool masks = FORM == 0 || (FORM == 2 && upper);
       const bool one_frame = FORM == 0 || (FORM == 2 && top);
+      // tiles of fewer than 16 candidates: the lane groups past them start at -inf
+      const float c0 = FORM == 2 && 4 * kg >= CRU ? -INFINITY : 0.f;
       const float* ccr = a.cosb + (int64_t)CR * HALF;  // the angle CR
       const float* scr = a.sinb + (int64_t)CR * HALF;
       auto nodes = [&](int bi, int (&nd)[UA]) {
@@ -553,13 +555,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
             load_k(KH, nd[j], kh[j]);
             load_k(KL, nd[j], kl[j]);
           }
-          f32x4 ci = {0.f, 0.f, 0.f, 0.f};
+          f32x4 ci = {c0, c0, c0, c0};
           if (masks) {  // -inf where the candidate is passed down
             const int p0 = tau << lgt;
             const uint32_t w = (uint32_t)uniform((int)selw[p0 >> 5]) >> (p0 & 31);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-              ci[r] = __int_as_float(__builtin_amdgcn_sbfe((int)w, 4 * kg + r, 1) & 0xff800000);
+              ci[r] = __int_as_float((__builtin_amdgcn_sbfe((int)w, 4 * kg + r, 1) & 0xff800000) |
+                                     (FORM == 2 ? __float_as_int(c0) : 0));
           }
           S[j] = ci;
 #pragma unroll
@@ -574,13 +577,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
         nodes(last || bi + NW >= nb ? bi : bi + NW, nn);
         if (PIPE) keys(nn);
         // S[j][r] = score[candidate 4kg + r of tile tau0 + j][g = u16]
-        if ((FORM != 0 && !wide) || last) {
+        if (last) {
 #pragma unroll
           for (int j = 0; j < UA; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              const int cu = 4 * kg + r;
-              const bool ok = tau0 + j < nt && cu < CRU && ((tau0 + j) << lgt) + cu < nc;
+              const bool ok = tau0 + j < nt && ((tau0 + j) << lgt) + 4 * kg + r < nc;
               S[j][r] = ok ? S[j][r] : -INFINITY;
             }
         }

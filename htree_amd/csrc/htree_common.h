@@ -93,12 +93,16 @@ struct Plan {
 
 // Dynamic LDS of the wide forward (byte offsets): both parent lists, the
 // selection bits, every tile's running max, block reduction slots, and the
-// importance of every candidate position (reused to merge the waves' states).
+// importance of every candidate position (reused to merge the waves' states);
+// `total` counts the static RoPE rows of its importance batches beside them.
 // A block of `parts` KV heads sharing one selection (2: a KV-head pair, 4: a
 // quad) keeps a running max and an importance array per part, and merges
 // each part's waves in a region of its own.
+constexpr int kWideBatch = 4;  // tiles of an importance batch
+// floats of a wave's table rows (D = 32: a cos and a sin row per tile)
+__host__ __device__ constexpr int wide_tab_floats(int D) { return D == 32 ? kWideBatch * D : 0; }
 struct WideLds {
-  int par, selw, mt, red, imp, merge_part, bytes;
+  int par, selw, mt, red, imp, merge_part, bytes, total;
 };
 __host__ __device__ inline WideLds wide_lds(int TK, int maxpos, int max_tiles, int D,
                                             int parts = 1) {
@@ -112,6 +116,7 @@ __host__ __device__ inline WideLds wide_lds(int TK, int maxpos, int max_tiles, i
   w.merge_part = 4 * (kWideWaves / parts) * 16 * (D + 3);  // a part's waves' states
   const int merge_bytes = w.merge_part * parts;
   w.bytes = w.imp + (imp_bytes > merge_bytes ? imp_bytes : merge_bytes);
+  w.total = w.bytes + 4 * kWideWaves * wide_tab_floats(D);
   return w;
 }
 

@@ -64,7 +64,7 @@ template <int D, bool PREC, typename TIn, bool TRACE, int C, int NH = 1, bool SE
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 && C == 32 ? 2 : 1))) void fwd_wide_kernel(const FwdArgs a) {
   static_assert(!(SEL && TRACE), "selection only: no trace");
   constexpr int KS = D / 32, ND = D / 16, HALF = D / 2;
-  constexpr int U = 4;                 // tiles of a batch: importance,
+  constexpr int U = kWideBatch;        // tiles of a batch: importance,
   constexpr int UA = D <= 64 ? 4 : 1;  // accumulation
   // D = 32: the next batch's keys (and the importance's table rows, through
   // LDS) are loaded while a batch is computed; D <= 64: a batch's values while
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
   float* imp0 = (float*)(lds + LO.imp);
   float* imp = imp0 + part * (TK << crlg);
 
-  __shared__ __attribute__((aligned(16))) float tab[kWideWaves][PIPE ? U * D : 1];  // table rows of a batch
+  __shared__ __attribute__((aligned(16))) float tab[kWideWaves][PIPE ? wide_tab_floats(D) : 1];  // table rows of a batch
 
   const int64_t grp = (int64_t)(blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
   if (grp >= (int64_t)a.B * a.Hkv * a.T / NH) return;  // uniform over the block

@@ -54,10 +54,10 @@ int make_plan(const htree_dims* d, Plan* p) {
   // selection.
   bool split = d->kv_share > 4 || npos > kWideMaxPos || d->top_k > kWideMaxTK;
   if (d->kv_share == 2 && wide &&
-      wide_lds(d->top_k, (int)npos, (int)max_tiles, d->D, 2).bytes > 160 * 1024)
+      wide_lds(d->top_k, (int)npos, (int)max_tiles, d->D, 2).total > 160 * 1024)
     split = true;
   if (d->kv_share == 4 &&
-      wide_lds(d->top_k, (int)npos, (int)max_tiles, d->D, 4).bytes > 160 * 1024)
+      wide_lds(d->top_k, (int)npos, (int)max_tiles, d->D, 4).total > 160 * 1024)
     split = true;
 
   memset(p, 0, sizeof(*p));

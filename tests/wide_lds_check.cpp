@@ -1,16 +1,24 @@
-// Host replay of fwd_wide_kernel's LDS addressing (htree_amd/csrc/htree_fwd.hip)
-// against the layout the launch allocates (wide_lds() of htree_common.h, the
-// same function the kernel and its launch call).  For every configuration
+// Host replay of fwd_wide_kernel's addressing (htree_amd/csrc/htree_fwd_wide.h)
+// against the LDS layout its launch allocates (wide_lds() of htree_common.h, the
+// function the kernel, its launch and make_plan call).  For every configuration
 // the library accepts on the wide path (top_k > 64 or more than 64 candidate
 // tiles; top_k <= 1024, top_k * CR <= 16384, CR in [4, 128], D in {32, 64, 128, 256};
-// 32 selection keys per thread up to 8192 positions, 64 above; with one
-// part, and with the two parts of a KV-head pair where their layout fits
-// 160 KB) and for every configuration with the four parts of a KV-head quad
-// (groups of 33..64 heads run the wide forward at any level size) where
-// their layout fits 160 KB, and every level shape (np parents, child index ct of the query), each LDS
-// index the kernel forms is checked to lie inside its region, and the
-// regions to lie inside the allocation without overlapping.  Test
-// infrastructure: built and run by tests/test_wide_lds.py on the CPU.
+// one part, and the two parts of a KV-head pair where their layout fits
+// 160 KB) and every configuration with the four parts of a KV-head quad
+// (any level size) where their layout fits 160 KB, and every level shape (np
+// parents, child index ct of the query), it forms each LDS index, list slot and
+// RoPE row of
+//   * the pass-down of a level of at most top_k candidates,
+//   * the importance batches (tiles clamped to the last one, the next batch's
+//     keys and table rows, the tab rows of D = 32),
+//   * the selection's keys (whole runs of C positions, of which only those below
+//     nc count), its list and bit writes,
+//   * the accumulation's batches in each form (slots past the list, the query
+//     turned back from them, the selection words), and the merge,
+// and checks it against its region where the value counts, against the
+// allocation where it is dropped.  The regions are disjoint and, with the
+// static rows, inside 160 KB.  Test infrastructure: built and run by
+// tests/test_wide_lds.py on the CPU.
 #include <cstdio>
 #include <cstdlib>
 
@@ -31,10 +39,6 @@ static int fails = 0;
     }                                                             \
   } while (0)
 
-struct Region {
-  long lo, hi;  // bytes [lo, hi)
-};
-
 static void check_config(int TK, int CR, int D, int parts) {
   int crlg = 0;
   while ((1 << crlg) < CR) ++crlg;
@@ -43,57 +47,100 @@ static void check_config(int TK, int CR, int D, int parts) {
   const WideLds w = wide_lds(TK, maxpos, max_tiles, D, parts);
   const int NW = kWideWaves / parts;                    // waves per part
   const int C = maxpos > kWideMidPos ? 2 * kWideC : kWideC;  // the launch's choice
-  const int WPT = C / 32;                                    // selection words per thread
-  CHECK(256 * C >= maxpos, "TK %d CR %d: %d keys per thread cover %d positions", TK, CR, C, maxpos);
+  const int U = kWideBatch, UA = D <= 64 ? 4 : 1;       // tiles of a batch
   const bool wide = CR >= 16;
-  const int CRU = CR < 16 ? CR : 16;
-  // regions as the kernel reads them
-  const Region par{w.par, (long)w.par + 2L * TK * 4};
-  const Region selw{w.selw, (long)w.selw + 256L * WPT * 4};  // selw[tid * WPT + j]
-  const Region mt{w.mt, (long)w.mt + (long)max_tiles * parts * 4};
-  const Region red{w.red, (long)w.red + 36L * 4};       // counts, scans, maxima
-  const long imp_floats = (w.bytes - w.imp) / 4;
-  const Region all{0, w.bytes};
-  const Region rs[4] = {par, mt, red, {w.imp, w.bytes}};
-  for (const Region& r : rs) CHECK(r.lo >= all.lo && r.hi <= all.hi, "TK %d CR %d D %d region", TK, CR, D);
-  CHECK(par.hi <= selw.lo, "TK %d CR %d: par / selw", TK, CR);
-  CHECK(w.selw + (maxpos + 31) / 32 * 4 <= mt.lo, "TK %d CR %d: selw / mt", TK, CR);
-  CHECK(mt.hi <= red.lo && red.hi <= w.red + 256 && w.red + 256 <= w.imp, "TK %d CR %d: mt / red / imp", TK, CR);
+  const int CRU = CR < 16 ? CR : 16, lgt = wide ? 4 : crlg;
+  const int rows = maxpos;  // RoPE rows make_plan asks for (and more than CR of them)
+  const int words = (maxpos + 31) / 32;
+  const long imp_floats = (w.bytes - w.imp) / 4, lds_floats_from_mt = (w.bytes - w.mt) / 4;
+  // ---- regions: par | selw | mt | red | imp, the static rows beside them
+  CHECK(256 * C >= maxpos, "TK %d CR %d: %d keys per thread", TK, CR, C);
+  CHECK(w.par == 0 && 2L * TK * 4 <= w.selw && w.selw + 4L * words <= w.mt, "par / selw / mt");
+  CHECK(w.mt + 4L * max_tiles * parts <= w.red && w.red + 256 <= w.imp, "mt / red / imp");
+  CHECK(4L * 36 <= 256, "red: counts, scans, maxima");
+  CHECK(4L * maxpos * parts <= w.bytes - w.imp, "importance of every part");
   CHECK(w.imp % 16 == 0 && w.mt % 4 == 0 && w.red % 4 == 0, "alignment");
-  // selection bits are written by threads with tid * C < maxpos only
-  for (int tid = 0; tid < 256; ++tid)
-    if (tid * C < maxpos)
-      CHECK(w.selw + (tid + 1) * WPT * 4 <= (long)w.selw + (maxpos + 31) / 32 * 4, "selw[%d]", tid);
-  (void)selw;
-  // every level shape: np valid parents, the query's child index ct
-  for (int np = 1; np <= TK; ++np)
-    for (int ct = 0; ct < CR; ++ct) {
-      const int nc = ((np - 1) << crlg) + ct + 1;
-      const int nt = wide ? (nc + 15) >> 4 : np;
-      CHECK(nc <= maxpos, "nc %d > maxpos %d", nc, maxpos);
-      CHECK(nt <= max_tiles, "TK %d CR %d: nt %d > max_tiles %d", TK, CR, nt, max_tiles);
-      // importance writes imp[pos], pos < nc; key reads imp[pos], mt[tile(pos)]
-      for (int tau = 0; tau < nt; ++tau) {
-        const int slot = wide ? (tau << 4) >> crlg : tau;
-        CHECK(slot < np, "slot %d of tile %d, np %d", slot, tau, np);
-        for (int u = 0; u < 16; ++u) {
-          const int pos = wide ? (tau << 4) + u : (tau << crlg) + u;
-          if (!(u < CRU && pos < nc)) continue;
-          for (int hf = 0; hf < parts; ++hf)  // the part's array, read by the keys of all parts
-            CHECK(hf * maxpos + pos < imp_floats, "imp[%d] of part %d of %ld", pos, hf, imp_floats);
-          CHECK((pos >> 5) < 256 * WPT && (pos >> 5) * 4 + 4 <= (maxpos + 31) / 32 * 4, "selw word of %d", pos);
-          const int mtile = wide ? pos >> 4 : pos >> crlg;
-          CHECK(mtile == tau && mtile < max_tiles, "mt index %d for tile %d", mtile, tau);
-          for (int hf = 0; hf < parts; ++hf)
-            CHECK(w.mt + (hf * max_tiles + mtile + 1) * 4 <= mt.hi, "mt of part %d", hf);
+  CHECK(w.total == w.bytes + (D == 32 ? 2048 : 0) && w.total <= 160 * 1024, "total %d", w.total);
+  CHECK(CR < rows || maxpos == CR, "row of the angle CR");  // (rope_rows > CR is a rule of its own)
+  // ---- tab (D = 32): element lane + 64 k of a wave's rows, read at D j (+ D / 2) + 8 (kg & 1) .. + 7
+  if (D == 32) {
+    CHECK((63 + 64 * (U * D / 64 - 1)) < wide_tab_floats(D), "tab write");
+    CHECK(D * (U - 1) + D / 2 + 8 + 7 < wide_tab_floats(D), "tab read");
+    for (int i = 0; i < U * D; ++i) CHECK(i / D < U, "tab row");
+  }
+  // ---- keys: thread tid reads positions C tid .. C tid + C - 1 of every part in 16-byte runs
+  for (int tid = 0; tid < 256; ++tid) {
+    if ((long)tid * C < maxpos)  // (the selection words it writes)
+      CHECK((tid + 1) * (C / 32) <= words, "selw of thread %d, maxpos %d", tid, maxpos);
+    for (int j = 0; j < parts; ++j)
+      for (int i4 = 0; i4 < C; i4 += 4) {
+        const int pos = tid * C + i4;
+        if ((long)tid * C >= maxpos) continue;  // tid * C < nc <= maxpos
+        CHECK((j * maxpos + pos) % 4 == 0, "16-byte run at %d", j * maxpos + pos);
+        CHECK(j * maxpos + pos + 3 < imp_floats, "TK %d CR %d D %d: imp run %d of part %d past the allocation",
+              TK, CR, D, pos, j);
+        CHECK(j * max_tiles + (pos >> lgt) < lds_floats_from_mt, "mt of run %d past the allocation", pos);
+        if (pos < maxpos) {  // a run with a candidate in it: one tile, this part's regions
+          CHECK((pos >> lgt) == ((pos + 3) >> lgt) && (pos >> lgt) < max_tiles, "run %d in one tile", pos);
+          CHECK(pos + 3 < maxpos, "run %d in the part's importances", pos);
         }
       }
-      // the select's parent reads pc[pos >> crlg] and list writes pn[idx], idx < take
-      const int take = TK < nc ? TK : nc;
-      CHECK(take <= TK, "take");
-      for (int pos = 0; pos < nc; ++pos) CHECK((pos >> crlg) < np, "pc index of %d", pos);
+  }
+  // ---- every level shape
+  for (int np = 1; np <= TK; ++np)
+    for (int ct = 0; ct < CR; ++ct) {
+      const int nc = ((np - 1) << crlg) + ct + 1, apos = nc - 1;
+      const int nt = wide ? (nc + 15) >> 4 : np;
+      CHECK(nc <= maxpos && nt <= max_tiles, "nc %d nt %d", nc, nt);
+      auto slot_of = [&](int tau) { return wide ? (tau << 4) >> crlg : tau; };
+      auto tile_ok = [&](int tau, const char* what) {
+        CHECK(tau >= 0 && tau < nt && slot_of(tau) < np, "%s: tile %d of %d, np %d", what, tau, nt, np);
+        // its first candidate exists, so its node's 16-node block does
+        CHECK((wide ? tau << 4 : tau << crlg) < nc, "%s: first candidate of tile %d", what, tau);
+      };
+      // a level passed down: pc[i >> crlg] of nc positions, nc <= TK entries written
+      if (nc <= TK) CHECK(((nc - 1) >> crlg) < np, "pass-down");
+      // importance
+      for (int wvh = 0; wvh < NW; ++wvh)
+        for (int i0 = wvh; i0 < nt; i0 += U * NW)
+          for (int j = 0; j < U; ++j) {
+            const int tau = i0 + NW * j < nt ? i0 + NW * j : nt - 1;
+            tile_ok(tau, "importance");
+            const int prow = apos - (slot_of(tau) << crlg);
+            CHECK(prow >= 0 && prow < rows, "row %d", prow);
+            const int nx = i0 + U * NW < nt ? i0 + U * NW : i0;
+            tile_ok(nx + NW * j < nt ? nx + NW * j : nt - 1, "next batch");
+          }
+      for (int tk = 0; tk < nt; ++tk) {  // stores: mt[tk], imp[(tk << lgt) + u] where a candidate
+        CHECK(tk < max_tiles, "mt store");
+        const int last = (tk << lgt) + CRU - 1 < nc ? (tk << lgt) + CRU - 1 : nc - 1;
+        CHECK(last < maxpos, "imp store");
+      }
+      // the selection: pn[idx] (idx < take), pc[pos >> crlg] (pos < nc)
+      CHECK((TK < nc ? TK : nc) <= TK && ((nc - 1) >> crlg) < np, "list");
+      // accumulation: batch bi of UA tiles by wave bi mod NW
+      const int nb = (nt + UA - 1) / UA;
+      for (int bi = 0; bi < nb; ++bi)
+        for (int j = 0; j < UA; ++j) {
+          const int tau0 = bi * UA, tau = tau0 + j < nt ? tau0 + j : nt - 1;
+          tile_ok(tau, "accumulation");
+          CHECK((tau << lgt) >> 5 < words, "selection word of tile %d", tau);
+          // one word holds the tile's bits (FORM 0 and 2)
+          CHECK((((tau << lgt) & 31) + CRU) <= 32, "bits of tile %d", tau);
+          // FORM 0 (whole tiles of the top level's nodes 0 .. apos)
+          if (UA > 1 && wide) CHECK(16 * tau <= apos, "top-level tile %d", tau);
+          // FORM 1 (CR 16, TK >= UA): slots past the list, and the rows turned back from them
+          if (UA > 1 && CR == 16 && TK >= UA) {
+            CHECK(tau0 + j < TK, "pc[%d] of %d", tau0 + j, TK);
+            const int prow = apos - ((tau0 + j) << crlg);
+            CHECK((prow < 0 ? -prow : prow) < rows, "row %d", prow);
+          }
+          // FORM 2
+          const int prow = apos - (slot_of(tau) << crlg);
+          CHECK(prow >= 0 && prow < rows, "row %d", prow);
+        }
     }
-  // each part's waves merge in the importance area, part hf from byte
+  // ---- each part's waves merge in the importance area, part hf from byte
   // merge_part * hf: mw, lw then ow rows of D + 1
   const int DP = D + 1;
   for (int hf = 0; hf < parts; ++hf) {
@@ -114,26 +161,24 @@ static void check_config(int TK, int CR, int D, int parts) {
 }
 
 int main() {
-  int n = 0;
+  int n = 0, refused = 0;
   for (int D : {32, 64, 128, 256})
     for (int CR = 4; CR <= 128; CR *= 2)
       for (int TK = 1; TK <= kWideMaxTK; TK *= 2) {
         if ((long)TK * CR > kWideMaxPos) continue;
         const int max_tiles = TK * (CR > 16 ? CR : 16) / 16;
         const bool wide = max_tiles > kMaxTiles || TK > kMaxTK;  // make_plan
-        // quads: any level size (make_plan's LDS rule)
-        if (wide_lds(TK, TK * CR, max_tiles, D, 4).bytes <= 160 * 1024) {
-          check_config(TK, CR, D, 4);
-          ++n;
-        }
-        if (!wide) continue;
-        check_config(TK, CR, D, 1);
-        ++n;
-        if (wide_lds(TK, TK * CR, max_tiles, D, 2).bytes <= 160 * 1024) {  // make_plan's rule
-          check_config(TK, CR, D, 2);
+        for (int parts : {1, 2, 4}) {
+          if (parts < 4 && !wide) continue;  // (quads: any level size)
+          const WideLds w = wide_lds(TK, TK * CR, max_tiles, D, parts);
+          // the static rows take no configuration from the wide form
+          refused += w.bytes <= 160 * 1024 && w.total > 160 * 1024;
+          if (parts > 1 && w.total > 160 * 1024) continue;  // make_plan: the split selection
+          check_config(TK, CR, D, parts);
           ++n;
         }
       }
+  CHECK(refused == 0, "%d layouts only fit without their static rows", refused);
   std::printf("%d wide configurations checked, %d failures\n", n, fails);
   return fails ? 1 : 0;
 }

@@ -91,13 +91,11 @@ int make_plan(const htree_dims* d, Plan* p) {
     p->off_vl[l] = p->precise ? take(elems) : -1;
     p->off_sh[l] = p->off_kh[l];
     p->off_sl[l] = p->off_kl[l];
-    const bool abs = wide_fwd && l == L - 1;
-    if (wide_fwd && (d->D == 32 || abs)) {
-      // read where the level selects, and by the stored-dS backward of quads
-      // (its K~^T is at the child's angle)
-      const bool needed = l > 0 || (abs && !wide);
-      p->off_sh[l] = needed ? take(elems) : -1;
-      p->off_sl[l] = needed ? take(elems) : -1;
+    const int second = tree_level_second(wide_fwd, wide, d->D, l, L);
+    if (second) p->off_sh[l] = p->off_sl[l] = -1;
+    if (second > 0) {
+      p->off_sh[l] = take(elems);
+      p->off_sl[l] = take(elems);
     }
   }
   p->pairs = wide_fwd || d->D != 32;

@@ -80,6 +80,18 @@ __host__ __device__ inline bool tree_level_abs(bool top_abs, int l, int L) {
   return top_abs && l == L - 1;
 }
 
+// Whether a level holds a K~ of its own for the scores that select (SH / SL:
+// the child's angle, dslot's order): 0 KH / KL serve, 1 it does, -1 nothing reads
+// one.  wide_fwd: the wide forward, whose top level's KH / KL are at the node's
+// angle and whose D = 32 ones are in pair order.  Read where a level selects
+// and, short (not wide) lists, by the stored-dS backward of quads (its K~^T is at
+// the child's angle).
+__host__ __device__ inline int tree_level_second(bool wide_fwd, bool wide, int D, int l, int L) {
+  const bool abs = tree_level_abs(wide_fwd, l, L);
+  if (!wide_fwd || (D != 32 && !abs)) return 0;
+  return l > 0 || (abs && !wide) ? 1 : -1;
+}
+
 // Element (d, node) of a level's V^T blocks: 16-node blocks of four 4-node
 // quads, (d, c) at (c / 4) * 4D + d * 4 + c % 4.
 __host__ __device__ inline int64_t tree_vt_index(int64_t Np, int D, int64_t bh, int64_t node,

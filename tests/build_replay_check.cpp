@@ -5,7 +5,8 @@
 // launch and the per-level launches, including level 1 pooled from the
 // leaves when CR > 64, partial spans and partial last parents) it checks:
 //   * every store lies inside its array, and every element of every packed
-//     array (K~ hi / lo rows, V^T blocks) and of every pooled level is
+//     array (K~ blocks in either element order, the second K~ of the levels that
+//     hold one, V^T blocks) and of every pooled level is
 //     written exactly once, padding rows included; the one exception is the
 //     level-0 V^T padding, which the last span and the zeroing block both
 //     write as zeros;
@@ -44,7 +45,9 @@ struct Arr {
   }
 };
 
-static void check_shape(int64_t T, int CR, int64_t MTN, int D, int BH) {
+// form: 0 the register, streaming and split forms, 1 the wide form, 2 quads of
+// short lists (make_plan's rules)
+static void check_shape(int64_t T, int CR, int64_t MTN, int D, int BH, int form) {
   int64_t N[16], Np[16], pw[16];
   int L = 0;
   if (!tree_level_sizes(T, CR, MTN, 16, N, &L)) return;
@@ -57,22 +60,46 @@ static void check_shape(int64_t T, int CR, int64_t MTN, int D, int BH) {
   }
   const int lspan = tree_lspan(L, pw);
   const int HALF = D / 2;
-  std::vector<Arr> kh(L), vh(L), lx(L);
+  const bool wide_fwd = form > 0, pairs = wide_fwd || D != 32;
+  std::vector<Arr> kh(L), sh(L), vh(L), lx(L);
   for (int l = 0; l < L; ++l) {
     kh[l].init(BH * Np[l] * D);
+    if (tree_level_second(wide_fwd, form == 1, D, l, L) > 0) sh[l].init(BH * Np[l] * D);
     vh[l].init(BH * Np[l] * D);
     lx[l].init(BH * N[l] * D);  // pooled level rows (levels >= 1), per (b, h_kv)
   }
-  auto pack_k = [&](int l, int64_t bh, int64_t nf, int cnt) {
+  auto pack_k_at = [&](int l, int64_t bh, int64_t nf, int cnt, bool abs, bool to_k, bool to_s) {
     for (int it = 0; it < cnt * (D / 8); ++it) {
       int j, i0;
       pack_k_item(it, D, &j, &i0);
       const int64_t row = tree_krow(Np[l], D, bh, nf + j);
       CHECK(nf + j < N[l], "pack_k node %lld of %lld", (long long)(nf + j), (long long)N[l]);
-      for (int q = 0; q < 4; ++q) {
-        kh[l].put(row + i0 + q, "kh", l);
-        kh[l].put(row + HALF + i0 + q, "kh", l);
+      // the table row of its angle: below CR, or of a top node, which lies
+      // below max_top_nodes (where the tree has more levels) and below T
+      const int64_t c = abs ? nf + j : (nf + j) & (CR - 1);
+      CHECK(c >= 0 && c < (abs ? (MTN > CR ? MTN : CR) : CR), "angle row %lld", (long long)c);
+      // 8-byte stores of four elements each
+      auto store = [&](Arr& a, int64_t o, const char* what) {
+        CHECK(o % 4 == 0, "%s store at %lld", what, (long long)o);
+        for (int q = 0; q < 4; ++q) a.put(o + q, what, l);
+      };
+      if (to_k) {
+        store(kh[l], tree_kindex(D, pairs, row + i0), "kh");
+        store(kh[l], tree_kindex(D, pairs, row + HALF + i0), "kh");
       }
+      if (to_s) {
+        store(sh[l], tree_kchunk(D, row + i0), "sh");
+        store(sh[l], tree_kchunk(D, row + HALF + i0), "sh");
+      }
+    }
+  };
+  auto pack_k = [&](int l, int64_t bh, int64_t nf, int cnt) {
+    const bool second = !sh[l].n.empty();
+    if (tree_level_abs(wide_fwd, l, L)) {
+      pack_k_at(l, bh, nf, cnt, true, true, false);
+      if (second) pack_k_at(l, bh, nf, cnt, false, false, true);
+    } else {
+      pack_k_at(l, bh, nf, cnt, false, true, second);
     }
   };
   auto pack_v = [&](int l, int64_t bh, int64_t nf, int cnt) {
@@ -100,7 +127,9 @@ static void check_shape(int64_t T, int CR, int64_t MTN, int D, int BH) {
       for (int l = 0; l < L; ++l)
         for (int64_t node = N[l]; node < Np[l]; ++node)
           for (int d = 0; d < D; ++d) {
-            kh[l].put(tree_krow(Np[l], D, bh, node) + d, "kh pad", l);
+            kh[l].put(tree_kindex(D, pairs, tree_krow(Np[l], D, bh, node) + d), "kh pad", l);
+            if (!sh[l].n.empty())
+              sh[l].put(tree_kchunk(D, tree_krow(Np[l], D, bh, node) + d), "sh pad", l);
             vh[l].put(tree_vt_index(Np[l], D, bh, node, d), "vt pad", l);
           }
     pack_k(0, bh, n0, nl);
@@ -155,7 +184,11 @@ static void check_shape(int64_t T, int CR, int64_t MTN, int D, int BH) {
     for (int64_t bh = 0; bh < BH; ++bh)
       for (int64_t node = 0; node < Np[l]; ++node)
         for (int d = 0; d < D; ++d) {
-          const int nk = kh[l].n[(size_t)(tree_krow(Np[l], D, bh, node) + d)];
+          const int64_t row = tree_krow(Np[l], D, bh, node) + d;
+          const int nk = kh[l].n[(size_t)tree_kindex(D, pairs, row)];
+          const int ns = sh[l].n.empty() ? 1 : sh[l].n[(size_t)tree_kchunk(D, row)];
+          CHECK(ns == 1, "T %lld CR %d D %d: sh level %d node %lld d %d written %d times",
+                (long long)T, CR, D, l, (long long)node, d, ns);
           const int nv = vh[l].n[(size_t)tree_vt_index(Np[l], D, bh, node, d)];
           const int want_v = (l == 0 && node >= N[0]) ? 2 : 1;
           CHECK(nk == 1, "T %lld CR %d D %d: kh level %d node %lld d %d written %d times",
@@ -179,7 +212,9 @@ int main() {
       for (int D : Ds)
         for (int64_t MTN : {1, 4, 16, 64, 256, 1024, 8192}) {
           if (D == 256 && T > 5000) continue;
-          check_shape(T, CR, MTN, D, 2);
+          // (the element order matters at D = 32, the top level's angle at every D)
+          for (int form : {0, 1, 2})
+            if (form == 0 || (D < 256 && T <= 5000)) check_shape(T, CR, MTN, D, 2, form);
         }
   std::printf("%ld shapes, %d failures\n", shapes, fails);
   return fails ? 1 : 0;

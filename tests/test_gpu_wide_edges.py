@@ -4,7 +4,7 @@ candidate down (at most top_k of them) and the first queries past that, a top
 level that is also the bottom one, three levels, batches of four tiles cut
 short (the bottom level's slots past the list), several tiles per slot and
 several slots per tile, padding heads.  The bars are those of the other
-forward tests (selection with its tie band, output by dtype)."""
+forward tests (selection with its tie band, output and softmax state by dtype)."""
 import pytest
 import torch
 
@@ -34,4 +34,4 @@ def test_wide_forms_against_oracle(B, T, H, Hkv, D, dtype, CR, TK, MTN):
                                                               MTN, TK)
     torch.cuda.synchronize()
     check_forward(q, k, v, CR, TK, MTN, dtype, out_dev=out.float().cpu().numpy(),
-                  parents_dev=par.cpu().numpy())
+                  parents_dev=par.cpu().numpy(), gmax_dev=gmax.cpu().numpy(), gsum_dev=gsum.cpu().numpy())

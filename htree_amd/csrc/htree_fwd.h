@@ -89,16 +89,13 @@ __device__ __forceinline__ void to_bf_split(const float (&x)[D / 32][8], bf16x8 
 // the level (m, l, O) is that level's own state (LayerTrace of
 // src/naive.py:13-19, filled at :225-227): max and output relative to the
 // max over the level's accumulated candidates, -1e10 / 0 / 0 where the level
-// accumulated nothing.  O[n][r] is output dim 16n + 4kg + r of head u16.
-// Output dim of row i of O tile n.  PERM (the register forward): tiles 2j
-// and 2j + 1 hold the even and the odd dims of 32j .. 32j + 31, so that the
-// V^T fragments of a tile pair are one 16-byte load.
-template <bool PERM>
-__device__ __forceinline__ int odim(int n, int i) {
-  return PERM ? 32 * (n >> 1) + 2 * i + (n & 1) : 16 * n + i;
-}
+// accumulated nothing.  O[n][r] is output dim odim(n, 4kg + r) of head u16.
+// Output dim of row i of O tile n: tiles 2j and 2j + 1 hold the even and the
+// odd dims of 32j .. 32j + 31, so that the V^T fragments of a tile pair are one
+// 16-byte load.
+__device__ __forceinline__ int odim(int n, int i) { return 32 * (n >> 1) + 2 * i + (n & 1); }
 
-// The head's output row from its O tiles (odim<true>): a lane's values of a
+// The head's output row from its O tiles (odim): a lane's values of a
 // tile pair are the 8 consecutive dims 32j + 8kg .. + 7, stored as 16 bytes
 // (against 2-byte stores: T 131072, 64/8 heads -1.3%; T 32768 within 0.3%).
 template <int D, typename TIn, typename F>
@@ -115,7 +112,7 @@ __device__ __forceinline__ void store_out(TIn* op, int kg, const f32x4 (&O)[D / 
   }
 }
 
-template <int D, bool PERM = false>
+template <int D>
 __device__ __forceinline__ void trace_store(const FwdArgs& a, int l, int64_t hq, bool gv, int kg,
                                             float m, float lpart, const f32x4 (&O)[D / 16]) {
   const float lt = add_xor32(add_xor16(lpart));
@@ -125,7 +122,7 @@ __device__ __forceinline__ void trace_store(const FwdArgs& a, int l, int64_t hq,
 #pragma unroll
   for (int n = 0; n < D / 16; ++n)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) op[odim<PERM>(n, 4 * kg + r)] = O[n][r];
+    for (int r = 0; r < 4; ++r) op[odim(n, 4 * kg + r)] = O[n][r];
   if (kg == 0) {
     a.tmax[lh] = m == -INFINITY ? kNegInfSentinel : m;
     a.tsum[lh] = lt;
@@ -136,7 +133,7 @@ __device__ __forceinline__ void trace_store(const FwdArgs& a, int l, int64_t hq,
 // src/naive.py:215-223 (a state counts only where its sum > 1e-10); returns
 // the merged sum, the merged max in m and output in O.  Reads back what this
 // lane's trace_store calls wrote.
-template <int D, bool PERM = false>
+template <int D>
 __device__ __forceinline__ float trace_merge(const FwdArgs& a, int64_t hq, bool gv, int kg,
                                              float& m, f32x4 (&O)[D / 16]) {
   float gm = kNegInfSentinel, gs = 0.f;
@@ -155,14 +152,14 @@ __device__ __forceinline__ float trace_merge(const FwdArgs& a, int64_t hq, bool 
 #pragma unroll
         for (int n = 0; n < D / 16; ++n)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) O[n][r] = O[n][r] * sg + op[odim<PERM>(n, 4 * kg + r)] * sc;
+          for (int r = 0; r < 4; ++r) O[n][r] = O[n][r] * sg + op[odim(n, 4 * kg + r)] * sc;
         gm = nm;
       } else {
         gs = ls;
 #pragma unroll
         for (int n = 0; n < D / 16; ++n)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) O[n][r] = op[odim<PERM>(n, 4 * kg + r)];
+          for (int r = 0; r < 4; ++r) O[n][r] = op[odim(n, 4 * kg + r)];
         gm = lm;
       }
     }

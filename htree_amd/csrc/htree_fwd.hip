@@ -42,9 +42,8 @@ namespace htree {
 // half's level max, f = exp(m_half - m_pair); both waves of the pair pass
 // the arrays in the same order, so both select the same nodes.
 template <int MAXSLOT>
-__device__ __forceinline__ void select_topk(const float* __restrict__ imp, const float* mt,
-                                            float Mrun, int nt, int nc, int apos, int TK,
-                                            bool wide, int crlg, int CR, int CRU,
+__device__ __forceinline__ void select_topk(const float* __restrict__ imp, int nt, int nc, int apos,
+                                            int TK, bool wide, int crlg, int CR, int CRU,
                                             const int32_t* par_cur, int32_t* par_next,
                                             unsigned long long* selmask, int lane,
                                             const float* __restrict__ imp2 = nullptr,
@@ -65,10 +64,6 @@ __device__ __forceinline__ void select_topk(const float* __restrict__ imp, const
           v = 1e6f;  // rightmost candidate always kept (src/naive.py:93)
         } else {
           v = imp2 ? imp[64 * sl + lane] * f1 + imp2[64 * sl + lane] * f2 : imp[64 * sl + lane];
-          if (mt) {
-            const float m = mt[tau];
-            if (m != Mrun) v *= expf(m - Mrun);
-          }
         }
         key[sl] = __float_as_uint(v) + 1u;
       }
@@ -352,12 +347,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
         const WaveLdsR& W0 = lds_all[wv & ~1];
         const WaveLdsR& W1 = lds_all[wv | 1];
         const float m0 = W0.lvl_max, m1 = W1.lvl_max, mp = fmaxf(m0, m1);
-        select_topk<4>(W0.imp, nullptr, mp, nt, nc, apos, TK, wide, crlg, CR, CRU, W.par[cur],
+        select_topk<4>(W0.imp, nt, nc, apos, TK, wide, crlg, CR, CRU, W.par[cur],
                        W.par[cur ^ 1], W.selmask, lane, W1.imp, expf(m0 - mp), expf(m1 - mp));
         __syncthreads();  // the partner has read this wave's importances
       } else {
         wave_sync();
-        select_topk<4>(W.imp, nullptr, M, nt, nc, apos, TK, wide, crlg, CR, CRU, W.par[cur],
+        select_topk<4>(W.imp, nt, nc, apos, TK, wide, crlg, CR, CRU, W.par[cur],
                        W.par[cur ^ 1], W.selmask, lane);
         wave_sync();
       }
@@ -473,14 +468,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       }
     }
     if (TRACE)
-      trace_store<D, true>(a, l, ((int64_t)b * a.T + t) * a.H + h * G + u16, gv, kg, m_run, l_part, O);
+      trace_store<D>(a, l, ((int64_t)b * a.T + t) * a.H + h * G + u16, gv, kg, m_run, l_part, O);
     cur ^= 1;
   }
 
   if constexpr (SEL) return;
   float lt;
   if (TRACE) {
-    lt = trace_merge<D, true>(a, ((int64_t)b * a.T + t) * a.H + h * G + u16, gv, kg, m_run, O);
+    lt = trace_merge<D>(a, ((int64_t)b * a.T + t) * a.H + h * G + u16, gv, kg, m_run, O);
   } else {
     lt = add_xor32(add_xor16(l_part));
   }

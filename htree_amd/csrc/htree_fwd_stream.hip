@@ -82,7 +82,7 @@ struct TileStage {
   }
   // V^T fragments: nodes c0 .. c0+3 (one quad, c0 % 4 == 0) of the staged
   // block, output tiles 2j and 2j + 1 at dims 32j + 2 u16 and 32j + 2 u16 + 1
-  // (odim<true>) in one 16-byte read: the 16 lanes of a lane group read 256
+  // (odim) in one 16-byte read: the 16 lanes of a lane group read 256
   // contiguous bytes (no bank conflicts)
   __device__ __forceinline__ void vread(s16x4 (&vh)[D / 16], s16x4 (&vl)[D / 16], int c0,
                                         int u16) const {
@@ -475,7 +475,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     }
     wait_copies();  // no copy into the slot is left in flight past the level
     if (TRACE)
-      trace_store<D, true>(a, l, ((int64_t)b * a.T + t) * a.H + h * G + u16, u16 < G, kg,
+      trace_store<D>(a, l, ((int64_t)b * a.T + t) * a.H + h * G + u16, u16 < G, kg,
                            m_run, l_part, O);
     cur ^= 1;
   }
@@ -484,7 +484,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // final normalisation (src/parallel.py:321-363): out = o / s
   float lt;
   if (TRACE) {
-    lt = trace_merge<D, true>(a, ((int64_t)b * a.T + t) * a.H + h * G + u16, u16 < G, kg, m_run, O);
+    lt = trace_merge<D>(a, ((int64_t)b * a.T + t) * a.H + h * G + u16, u16 < G, kg, m_run, O);
   } else {
     lt = add_xor32(add_xor16(l_part));
   }

@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
         f32x4 z[ND];
 #pragma unroll
         for (int n = 0; n < ND; ++n) z[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-        trace_store<D, true>(a, l, hq, gv, kg, -INFINITY, 0.f, z);
+        trace_store<D>(a, l, hq, gv, kg, -INFINITY, 0.f, z);
       }
       cur ^= 1;
       continue;
@@ -521,9 +521,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
           const int tau = tau0 + j < nt ? tau0 + j : nt - 1;
           if (!one_frame) {
             const int s = FORM == 1 ? tau0 + j : slot_of(tau);
-            // (D >= 128: from the table at every slot, as turning on would
-            // hold the query twice and the angle's row in registers)
-            if (j == UA - 1 || (D >= 128 && (FORM == 1 || s != cs))) {
+            // (D >= 128, batches of one tile: from the table at every slot, as
+            // turning on would hold the query twice and the angle's row in registers)
+            if (j == UA - 1) {
               const int prow = apos - (s << crlg);
               if (FORM == 1 && prow < 0) {
                 // a slot past the list (the last batch turns back from it):
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
       float Ml, Ll;
       f32x4 Ol[ND];
       merge_waves(Ml, Ll, Ol);
-      if (wvh == 0) trace_store<D, true>(a, l, hq, gv, kg, Ml, kg == 0 ? Ll : 0.f, Ol);
+      if (wvh == 0) trace_store<D>(a, l, hq, gv, kg, Ml, kg == 0 ? Ll : 0.f, Ol);
     }
     cur ^= 1;
   }
@@ -664,7 +664,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 &&
   float M, lt;
   if (TRACE) {
     if (wvh != 0) return;
-    lt = trace_merge<D, true>(a, hq, gv, kg, M, O);
+    lt = trace_merge<D>(a, hq, gv, kg, M, O);
   } else {
     merge_waves(M, lt, O);
     if (wvh != 0) return;

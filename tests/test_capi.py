@@ -172,6 +172,34 @@ def test_workspace_too_small_rejected():
     assert rc == N.HTREE_EWORKSPACE
 
 
+def test_tree_workspace_holds_no_unread_copy():
+    """K~ hi and lo and V^T (hi, and lo for 16-bit-split types) of every level,
+    and a second K~ only where the wide forward selects from one of another
+    angle (the top level) or element order (D = 32)."""
+    up = lambda x, m: -(-x // m) * m
+
+    def want(T, H, Hkv, D, CR, TK, MTN, dtype, second):
+        n = level_sizes(T, CR, MTN)
+        b = lambda x: up(Hkv * up(x, 16) * D * 2, 256)
+        return (sum(b(x) for x in n) * (3 if dtype == torch.bfloat16 else 4)
+                + sum(2 * b(n[l]) for l in second(len(n))))
+
+    none, top, upper = lambda L: [], lambda L: [L - 1], lambda L: range(1, L)
+    for T, D, CR, TK, MTN, dtype, second in (
+            (5000, 32, 16, 16, 128, torch.bfloat16, none),   # register form
+            (5000, 32, 16, 16, 128, torch.float32, none),
+            (5000, 32, 32, 32, 256, torch.float16, none),    # streaming form
+            (5000, 128, 32, 32, 256, torch.bfloat16, none),
+            (5000, 32, 4, 2048, 8192, torch.float32, none),  # split selection
+            (5000, 32, 16, 512, 8192, torch.float32, none),  # wide form, one level
+            (5000, 64, 16, 512, 8192, torch.bfloat16, none),
+            (5000, 64, 16, 128, 128, torch.bfloat16, top),   # wide form, three levels
+            (5000, 32, 16, 128, 128, torch.float32, upper)):
+        d = dims(T=T, H=16, H_kv=2, D=D, compression_rate=CR, top_k=TK, max_top_nodes=MTN, dtype=dtype,
+                 rope_rows=TK * CR)
+        assert N.tree_workspace_bytes(d) == want(T, 16, 2, D, CR, TK, MTN, dtype, second), (T, D, TK)
+
+
 def test_python_api_validates_like_reference():
     import htree_amd
     from htree_amd.parallel import HeadFrame

@@ -423,6 +423,9 @@ def main():
         "roofline": {
             "kernel": f"htree::{forward_kernel(args.workload)} (fused forward, all levels)",
             "bound": "hbm",
+            "bound_note": "frac is gathered bytes over the HBM peak, the target's measure; L2 and "
+                          "the MALL serve most of them (traffic: bytes beyond L2), so above 1 "
+                          "it is no bound",
             "achieved": achieved / 1e9,
             "peak": HBM_PEAK / 1e9,
             "unit": "GB/s",

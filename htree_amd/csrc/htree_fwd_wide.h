@@ -31,12 +31,15 @@ namespace htree {
 //     query; below, the query takes a batch's last slot from the table and
 //     turns by CR per slot.
 // Each wave keeps its own softmax state; they are merged at the end.
-// D = 32 is bound by the vector data path (72% busy: 2.0 TB of operands a
-// launch at T 120000, 64/4 heads, top_k 512) beside 59% of the vector ALU:
-// 240 -> 133 ms there, 24.0 -> 17.3 ms with 64 heads over one KV head at
-// D = 64, 23.8 -> 10.0 ms at D = 128, T 16000, top_k 256 (bf16).  Two waves per
-// SIMD: at three the batches' operands spill, and the spills cost more of the
-// same path (165 ms).
+// D = 32 is bound by the vector data path (71% busy: 2.0 TB of operands a
+// launch at T 120000, 64/4 heads, top_k 512) beside 58% of the vector ALU:
+// 240 -> 133 ms there against one tile at a time, 24.0 -> 18.5 ms with 64 heads
+// over one KV head at D = 64, 23.8 -> 10.2 ms at D = 128, T 16000, top_k 256
+// (bf16).  Two waves per SIMD.  Split operands at D <= 64 spill there already
+// (C = 32, 1 / 2 / 4 parts: D 32 fp32 24 / 29 / 43 VGPRs, D 64 fp32 35 / 42 /
+// 45; bf16 4 to 11), which takes the same path: 12 GB written per launch at
+// D = 32, 1 GB of it outputs.  At three waves more of the batches' operands
+// spill and it is slower (165 ms).
 // NH > 1 (kv_share 2 or 4: query groups of 17..32 or 33..64 heads): the
 // block takes KV heads NH h' .. NH h' + NH - 1 of one query (their keys and
 // values are the same), the kWideWaves / NH waves of part i the heads of KV
